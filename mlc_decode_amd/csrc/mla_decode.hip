@@ -2454,9 +2454,17 @@ template hipError_t launch_ws_dense<MLA_DTYPE_F16>(const KParams&, int, hipStrea
 #else
 
 // ---------------------------------------------------------------------------------------
-// paged KV-cache append: one wave per sequence (its length is read once, before its rows are
-// written, and advanced after them); lanes 0..63 copy the 512 latent dims and lanes 0..7
-// the 64 rope dims of each new row, 16 bytes per lane
+// paged KV-cache append.  SW waves of one workgroup share a sequence, wave w taking its new
+// tokens w, w + SW, ..; lanes 0..63 copy (or quantise) the 512 latent dims and lanes 0..7 the 64
+// rope dims of a row, 16 bytes per lane.  Every wave reads the length and checks all of the
+// sequence's pages at once (lane t holds the page of token t), and the length is advanced after
+// the workgroup barrier that follows, so one launch does both.  The call is a chain of memory
+// round trips (length, page ids, rows), so the rows are requested before the length arrives and
+// a wave holds at most four of them; one wave per sequence walked its tokens one after another,
+// a round trip each (kernel time: 32 sequences x 64 tokens into the fp8 cache 51.4 -> 7.4 us, one
+// sequence x 64 bf16 tokens 30.2 -> 3.7 us; 8192 pages quantised 264 -> 188 us, 5.0 TB/s).
+// The fp8 scales of a sequence go out through LDS, one wave per 128-dim block: consecutive tokens
+// are consecutive floats of a page's scale row.
 // ---------------------------------------------------------------------------------------
 struct AppendParams {
   const uint16_t* kv_new;
@@ -2486,42 +2494,59 @@ __device__ __forceinline__ int fp8_block_exp(uint32_t bits) {
   return k < -126 ? -126 : (k > 127 ? 127 : k);
 }
 
-__global__ __launch_bounds__(256) void mla_kv_append_kernel(AppendParams a) {
-  const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
+template <int SW>
+__global__ __launch_bounds__(SW == 16 ? 1024 : 256) void mla_kv_append_kernel(AppendParams a) {
+  constexpr int kSeqs = SW == 1 ? 4 : 1;         // sequences per workgroup
+  constexpr int kTok = SW == 16 ? 4 : 1;         // tokens per wave
+  static_assert(SW * kTok <= kPageTokens, "lane t holds the page of token t");
+  __shared__ float scale_sh[SW == 16 ? 4 : 1][kPageTokens];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  if (b >= a.batch) return;  // whole waves only
-  const int L = a.seqlens[b];
-  bool ok = L >= 0;
-  for (int t = 0; t < a.n_new; ++t) {
-    const int pos = L + t;
-    const int pi = pos >> 6;
-    if (pi >= a.max_pages) {
-      ok = false;
-    } else {
-      const int pg = a.block_table[(int64_t)b * a.bt_stride + pi];
-      ok = ok && pg >= 0 && pg < a.num_blocks;
+  const int b = blockIdx.x * kSeqs + (SW == 1 ? wave : 0);
+  const int w = SW == 1 ? 0 : wave;  // this wave's first token
+  if (b >= a.batch) return;  // whole waves only (SW == 1), or never
+  // the rows do not depend on the length or the pages: requested first
+  const uint16_t* src = a.kv_new + b * a.n_sb;
+  i32x4 v[kTok], r[kTok];
+#pragma unroll
+  for (int i = 0; i < kTok; ++i) {
+    const int t = w + SW * i;
+    if (t < a.n_new) {  // uniform
+      v[i] = *(const i32x4*)(src + t * a.n_st + 8 * lane);
+      if (lane < 8) r[i] = *(const i32x4*)(src + t * a.n_st + kRopeOff + 8 * lane);
     }
   }
-  if (!ok) {
-    if (lane == 0 && a.status != nullptr) a.status[0] = 1;
-    return;
+  const int L = a.seqlens[b];
+  const int pos_l = (int)((uint32_t)L + (uint32_t)lane);  // token `lane`'s position
+  int page = -1;
+  if (lane < a.n_new && L >= 0 && pos_l >= 0 && (pos_l >> 6) < a.max_pages)
+    page = a.block_table[(int64_t)b * a.bt_stride + (pos_l >> 6)];
+  const bool bad = lane < a.n_new && (page < 0 || page >= a.num_blocks);
+  const bool ok = __builtin_amdgcn_ballot_w64(bad) == 0;  // uniform, the same in every wave
+  if constexpr (SW > 1) __syncthreads();  // every wave has read the length
+  if (w == 0 && lane == 0) {
+    if (ok)
+      a.seqlens[b] = L + a.n_new;
+    else if (a.status != nullptr)
+      a.status[0] = 1;
   }
-  for (int t = 0; t < a.n_new; ++t) {
-    const int pos = L + t;
-    const int pg = a.block_table[(int64_t)b * a.bt_stride + (pos >> 6)];
-    const int row = pos & 63;
-    const uint16_t* src = a.kv_new + b * a.n_sb + t * a.n_st;
-    const i32x4 v = *(const i32x4*)(src + 8 * lane);
+  if (!ok) return;
+#pragma unroll
+  for (int i = 0; i < kTok; ++i) {
+    const int t = w + SW * i;
+    if (t >= a.n_new) break;  // uniform
+    const int pg = __builtin_amdgcn_readlane(page, t);
+    const int row = (L + t) & 63;
     if (a.kv8) {  // uniform
       // lane l holds dims 8l .. 8l+7; block j (dims 128j ..) is the lane group of 16
       float x[8];
       float amax = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int w = v[i];
-        x[2 * i] = __uint_as_float((uint32_t)w << 16);
-        x[2 * i + 1] = __uint_as_float((uint32_t)w & 0xFFFF0000u);
-        amax = fmaxf(amax, fmaxf(fabsf(x[2 * i]), fabsf(x[2 * i + 1])));
+      for (int j = 0; j < 4; ++j) {
+        const int c = v[i][j];
+        x[2 * j] = __uint_as_float((uint32_t)c << 16);
+        x[2 * j + 1] = __uint_as_float((uint32_t)c & 0xFFFF0000u);
+        amax = fmaxf(amax, fmaxf(fabsf(x[2 * j]), fabsf(x[2 * j + 1])));
       }
 #pragma unroll
       for (int m = 8; m >= 1; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 16));
@@ -2533,18 +2558,25 @@ __global__ __launch_bounds__(256) void mla_kv_append_kernel(AppendParams a) {
       hi = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_ldexpf(x[6], -k), __builtin_ldexpf(x[7], -k), hi, true);
       uint8_t* dst = (uint8_t*)a.kv_nope + (int64_t)pg * a.kv_sp + (int64_t)row * a.kv_st + 8 * lane;
       *(i32x2*)dst = i32x2{lo, hi};
-      if ((lane & 15) == 0)
-        a.kv_scale[(int64_t)pg * a.ks_sp + (int64_t)(lane >> 4) * a.ks_sb + row] =
-            __uint_as_float((uint32_t)(k + 127) << 23);
+      if ((lane & 15) == 0) {
+        const float sc = __uint_as_float((uint32_t)(k + 127) << 23);
+        if constexpr (SW == 16)
+          scale_sh[lane >> 4][t] = sc;
+        else
+          a.kv_scale[(int64_t)pg * a.ks_sp + (int64_t)(lane >> 4) * a.ks_sb + row] = sc;
+      }
     } else {
-      *(i32x4*)(a.kv_nope + (int64_t)pg * a.kv_sp + (int64_t)row * a.kv_st + 8 * lane) = v;
+      *(i32x4*)(a.kv_nope + (int64_t)pg * a.kv_sp + (int64_t)row * a.kv_st + 8 * lane) = v[i];
     }
-    if (lane < 8) {
-      const i32x4 r = *(const i32x4*)(src + kRopeOff + 8 * lane);
-      *(i32x4*)(a.kv_rope + (int64_t)pg * a.kr_sp + (int64_t)row * a.kr_st + 8 * lane) = r;
+    if (lane < 8) *(i32x4*)(a.kv_rope + (int64_t)pg * a.kr_sp + (int64_t)row * a.kr_st + 8 * lane) = r[i];
+  }
+  if constexpr (SW == 16) {
+    if (a.kv8) {  // uniform over the workgroup
+      __syncthreads();
+      if (wave < 4 && lane < a.n_new)
+        a.kv_scale[(int64_t)page * a.ks_sp + (int64_t)wave * a.ks_sb + (pos_l & 63)] = scale_sh[wave][lane];
     }
   }
-  if (lane == 0) a.seqlens[b] = L + a.n_new;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -4110,8 +4142,15 @@ int mla_kv_append(const mla_kv_append_args* a, void* stream) {
   k.kv8 = kv8 ? 1 : 0;
   k.kv_scale = a->kv_scale;
   k.ks_sp = a->kv_scale_stride_page; k.ks_sb = a->kv_scale_stride_blk;
-  hipLaunchKernelGGL(mla::mla_kv_append_kernel, dim3((a->batch + 3) / 4), dim3(256), 0,
-                     (hipStream_t)stream, k);
+  // waves per sequence: as few as hold a wave's tokens to one row (up to 4 new tokens), then 16
+  // waves of up to 4 rows each, all in flight together
+  const hipStream_t st = (hipStream_t)stream;
+  if (a->n_new == 1)
+    hipLaunchKernelGGL(mla::mla_kv_append_kernel<1>, dim3((a->batch + 3) / 4), dim3(256), 0, st, k);
+  else if (a->n_new <= 4)
+    hipLaunchKernelGGL(mla::mla_kv_append_kernel<4>, dim3(a->batch), dim3(256), 0, st, k);
+  else
+    hipLaunchKernelGGL(mla::mla_kv_append_kernel<16>, dim3(a->batch), dim3(1024), 0, st, k);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MLA_ERR_HIP, std::string("kv append launch failed: ") + hipGetErrorString(e));
   return MLA_OK;

@@ -81,6 +81,25 @@ def test_fp8_append_matches_oracle(gpu, n_new):
     assert_fp8_equal(cache, lat2, sc2, rope2, f"append n_new={n_new}")
 
 
+@pytest.mark.parametrize("n_new", [4, 17, 64])
+def test_fp8_append_many_tokens(gpu, n_new):
+    """Several waves per sequence; the scales of a sequence cross pages."""
+    torch.manual_seed(30 + n_new)
+    nb, B = 16, 4
+    lat, sc, rope = F8.quantize_pages(varied_cache(nb, n_new))
+    table = torch.randperm(nb).reshape(B, 4).to(torch.int32)
+    lens = torch.tensor([0, 63, 64, 150], dtype=torch.int32)
+    new = varied_cache(B, 200 + n_new).reshape(B, 64, 576)[:, :n_new].contiguous()
+    cache = to_gpu_fp8(lat, sc, rope)
+    lens_d = lens.cuda()
+    say(f"fp8 append many tokens n_new={n_new}")
+    kv_append(new.cuda(), cache, table.cuda(), lens_d)
+    torch.cuda.synchronize()
+    lat2, sc2, rope2, lens2 = F8.append_paged_fp8(lat, sc, rope, table, lens, new)
+    assert torch.equal(lens_d.cpu(), lens2)
+    assert_fp8_equal(cache, lat2, sc2, rope2, f"append many n_new={n_new}")
+
+
 def fp8_inputs(cfg, seed, quantize_on_gpu=False):
     """(inputs, fp8 cache on the GPU, dequantised fp32 cache for the oracle).  Large caches
     are quantised on the GPU (its quantiser is checked bit-exact against the oracle above)

@@ -568,6 +568,23 @@ def test_kv_append_matches_oracle(gpu, dtype, n_new):
         assert st.item() == 0
 
 
+@pytest.mark.parametrize("n_new", [4, 5, 16, 17, 33, 64])
+def test_kv_append_many_tokens(gpu, n_new):
+    """Several waves per sequence (at most one row each up to 4 tokens, then up to four): bit-exact
+    rows, a sequence past its table and one with a bad page id left untouched."""
+    cache, bt, lens, new = _append_inputs(60 + n_new, [0, 1, 63, 64, 130, 5 * 64 - 3, 100], n_new, 5, torch.bfloat16)
+    bt[6, (100 + n_new - 1) // 64] = -1
+    want_cache, want_lens, skipped = R.append_paged(cache, bt, lens, new)
+    assert skipped == [5, 6]
+    say(f"kv_append many tokens n_new={n_new}")
+    c, ln = cache.to(gpu), lens.to(gpu)
+    st = torch.zeros(1, dtype=torch.int32, device=gpu)
+    kv_append(new.to(gpu), c, bt.to(gpu), ln, status=st)
+    torch.cuda.synchronize()
+    assert st.item() == 1
+    assert torch.equal(c.cpu(), want_cache) and torch.equal(ln.cpu(), want_lens)
+
+
 def test_kv_append_skips_unassigned_pages(gpu):
     cache, bt, lens, new = _append_inputs(7, [10, 4 * 64 - 1, 64, 63, 5], 2, 4, torch.bfloat16)
     bt[3, 1] = cache.shape[0]  # sequence 3 crosses into a page id past the cache
