@@ -57,6 +57,8 @@ constexpr float kLog2e = 1.44269504088896340736f;
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef i32x2 i32x2_a4 __attribute__((aligned(4)));  // vectors at addresses of less alignment
+typedef i32x4 i32x4_a8 __attribute__((aligned(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short i16x4 __attribute__((__vector_size__(4 * sizeof(short))));
 typedef __bf16 bf16x8 __attribute__((__vector_size__(8 * sizeof(__bf16))));
@@ -2730,6 +2732,18 @@ __device__ __forceinline__ float merge_few_splits(const uint16_t* __restrict__ w
   return lse2;
 }
 
+// The merge of one row of 16-bit partials by one wave, by its number of splits.  (A queue of eight
+// rows in flight for 9 .. 64 splits, its waits counted per row, was no faster than the general
+// loop: 12.6 against 12.4 us in the absorb kernel, 7.0 against 7.0 us in the combine.)
+template <int DT, bool SCALED>
+__device__ __forceinline__ float merge_row16(const uint16_t* __restrict__ ws_o, const float* __restrict__ ws_scale,
+                                             const float* __restrict__ ws_lse, int base, int n, int rows, int row,
+                                             int lane, float* w_sh, float (&acc)[8]) {
+  if (n <= kFewSplits)  // uniform
+    return merge_few_splits<DT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, lane, acc);
+  return merge_splits_wave<DT, uint16_t, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, lane, w_sh, acc);
+}
+
 // merge_splits_wave for a row of at most kDeepSplits 16-bit partials, by four waves that each
 // take one 128-dim quarter q of the row (lane l: dims 128 q + 2 l, +1), so a long merge runs on
 // four CUs instead of one.  A wave keeps kQueue quarter rows in flight in a register queue: the
@@ -2886,10 +2900,7 @@ __global__ __launch_bounds__(DEEP ? 64 : 256) void mla_combine_kernel(const PT* 
   float acc[8];
   float lse2;
   if constexpr (std::is_same<PT, uint16_t>::value) {
-    if (n <= kFewSplits)  // uniform
-      lse2 = merge_few_splits<DT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, lane, acc);
-    else
-      lse2 = merge_splits_wave<DT, PT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, lane, w_sh, acc);
+    lse2 = merge_row16<DT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, lane, w_sh, acc);
   } else {
     lse2 = merge_splits_wave<DT, PT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, lane, w_sh, acc);
   }
@@ -2903,24 +2914,19 @@ __global__ __launch_bounds__(DEEP ? 64 : 256) void mla_combine_kernel(const PT* 
 // ---------------------------------------------------------------------------------------
 // v[m, h, :] = o[m, h, :] . W_UV[h]  (m = b * s_q + s, o the merged latent output, W_UV[h] the
 // head's 512 x kVDim up-projection, given k-blocked: w_blk[h][kb][n][kk] = W_UV[h][32kb + kk][n],
-// so the B operand of one MFMA k-step for 16 columns is one contiguous KiB).  One workgroup of
-// 4 waves per (head, tile of 16 rows); wave w merges rows 4w .. 4w+3 and owns output columns
-// 32w .. 32w+31.  The kernel is a chain of dependent memory round trips, so it is arranged to
-// have few:
-//  1. the rows' split ranges are loaded;
-//  2. the lse of each row's first 64 splits and the partial rows of its first kPF splits are
-//     loaded together (the partials do not depend on the weights); the rows are merged into LDS
-//     as bf16, never written to HBM (a single-split row is read from `out`, where the decode
-//     wrote it).  Each row follows the combine's arithmetic operation for operation
-//     (merge_splits_wave): the same lse (lane-strided max and sum, xor-butterfly), the same
-//     weights, the same fma chain in split order;
-//  3. the wave's W_UV slab (32 columns, 128 registers) is loaded in one round trip and 2 MFMA
-//     tiles form the 16 x kVDim product.
-// At most 256 registers (178 used): two workgroups per CU.  At three (168 registers) the
-// compiler spilled 28 of them to scratch and the kernel ran 4-21% slower.  (Measured
-// alternatives: loading W_UV before the merge, and 32-row workgroups of 8 waves that preload
-// their 16-column slabs, were no faster; the [h][n][k] layout, 16 half-lines per load, cost
-// 3 us more at 128 heads x 64 rows.)
+// so the fragment of one MFMA k-step for 16 columns is one contiguous KiB).  One workgroup of 16
+// waves per (head, tile of 16 rows); wave i merges row i and owns 16 output columns over one half
+// of the 512-dim contraction.  The kernel is bound by dependent memory round trips (split range,
+// then lse and partial rows), so it is arranged to have few and to keep them full:
+//  1. the wave's W_UV fragments (8 k-steps, 32 registers) are requested before anything else;
+//  2. its row is merged by the combine's own routines (merge_row16: the same bits as the combine
+//     kernel stores) into LDS in the input dtype, never to HBM (a single-split row is read from
+//     `out`, where the decode wrote it);
+//  3. eight MFMAs per wave form v^T tiles (W as the A operand, so that a lane holds four
+//     consecutive columns of a row); the two contraction halves are summed through LDS.
+// Four waves of four rows each, two splits a round trip, left 32 KiB in flight per CU and walked the
+// longest row's splits two at a time: 32 ragged sequences x 128 heads in 256 splits 29.6 -> 12.4 us
+// (38 MB of partials and 17 MB of weights: 4.4 TB/s).
 constexpr int kVDim = 128;
 constexpr int kAbsRows = 16;
 struct AbsorbParams {
@@ -2938,177 +2944,62 @@ struct AbsorbParams {
 };
 
 template <int DT>
-__global__ __launch_bounds__(256, 2) void mla_combine_absorb_kernel(AbsorbParams a) {
-  constexpr int RT = kAbsRows;     // rows per workgroup
-  constexpr int kPitch = kDV + 8;  // 16-bit elements; 1040-byte rows keep the A reads conflict-free
-  constexpr int R = RT / 4;        // rows merged by one wave
-  constexpr int NT = 2;            // 16-column MFMA tiles per wave
-  constexpr int KS = kDV / 32;     // MFMA k-steps
-  constexpr int kPF = 2;           // partial rows per row loaded in one round trip
-  // a group of kPF splits must not cross a 64-split weight window (w_sh holds one window);
-  // 4 spills 61 registers at this launch bound
-  static_assert(64 % kPF == 0, "kPF divides the weight window");
-  __shared__ __attribute__((aligned(16))) uint16_t a_sh[RT * kPitch];
-  __shared__ float w_sh[RT][64];
+__global__ __launch_bounds__(64 * kAbsRows) void mla_combine_absorb_kernel(AbsorbParams a) {
+  constexpr int kPitch = kDV + 8;       // 16-bit elements; 1040-byte rows keep the fragment reads conflict-free
+  constexpr int NT = kVDim / 16;        // 16-column tiles
+  constexpr int KS = kDV / 32 / 2;      // MFMA k-steps of one contraction half
+  static_assert(2 * NT == kAbsRows, "one wave per row, and per (column tile, contraction half)");
+  __shared__ __attribute__((aligned(16))) uint16_t a_sh[kAbsRows * kPitch];
+  __shared__ float w_sh[kAbsRows][64];
+  __shared__ f32x4 c_sh[NT][64];
   const int h = blockIdx.x;
-  const int m0 = blockIdx.y * RT;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, li = lane & 15;
+  const int nt = wave & (NT - 1), kh = wave / NT;
 
-  // ---- 1. split ranges of the wave's rows
-  const int r0 = wave * R;
-  const int64_t split_stride = (int64_t)a.rows * kDV;
-  int n[R];
-  const uint16_t* src1[R];  // single-split rows: the decode's output (input dtype)
-  const uint16_t* src[R];   // split rows: scaled fp16 partials
-  const float* scp[R];      // their scales (this lane's chunk, lane / 16)
-  const float* lsep[R];
-  int nmax = 0;
+  // ---- 1. W_UV fragments: 8 consecutive k of column 16 nt + li
+  const uint16_t* wb = a.w_blk + (((int64_t)h * (2 * KS) + kh * KS) * kVDim + 16 * nt + li) * 32 + 8 * g;
+  i32x4 wf[KS];
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int m = m0 + r0 + i;
-    n[i] = 0;
-    src1[i] = a.out;
-    src[i] = a.ws_o;
-    scp[i] = a.ws_scale;
-    lsep[i] = a.ws_lse;
-    if (m < a.m_rows) {
-      const int b = m / a.s_q, s = m - b * a.s_q;
-      const int row = s * a.heads + h;
-      const int base = a.splits[b];
-      n[i] = a.splits[b + 1] - base;
-      if (a.premerged && n[i] > 1) n[i] = 1;  // the merged row is in `out`, its lse written
-      if (n[i] == 1) {
-        src1[i] = a.out + b * a.o_sb + s * a.o_ss + h * a.o_sh + lane * 8;
-      } else {
-        src[i] = a.ws_o + ((int64_t)base * a.rows + row) * kDV + lane * 8;
-        scp[i] = a.ws_scale + ((int64_t)base * a.rows + row) * 4 + (lane >> 4);
-        lsep[i] = a.ws_lse + (int64_t)base * a.rows + row;
-      }
-    }
-    nmax = n[i] > nmax ? n[i] : nmax;
-  }
-  // the eight values of split u of row i owned by this lane, widened to fp32, and their scale
-  // (1 for a single-split row; branches are wave-uniform: all lanes work on the same row)
-  auto load_row = [&](int u, int i, float (&xv)[8], float& us) __attribute__((always_inline)) {
-    if (n[i] == 1) {
-      cvt8<DT>(*(const i32x4*)src1[i], xv);
-      us = 1.f;
-    } else {
-      load8<MLA_DTYPE_F16>(src[i] + u * split_stride, xv);
-      us = scp[i][(int64_t)u * a.rows * 4];
-    }
-  };
+  for (int ks = 0; ks < KS; ++ks) wf[ks] = *(const i32x4*)(wb + ks * kVDim * 32);
 
-  // ---- 2. partial rows of the first kPF splits, and the lse of split `lane`, in one round trip
-  float x[kPF][R][8], us[kPF][R];
-#pragma unroll
-  for (int u = 0; u < kPF; ++u)
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-      if (u < n[i]) load_row(u, i, x[u][i], us[u][i]);
-  float l0[R], lse2[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) l0[i] = (n[i] > 1 && lane < n[i]) ? lsep[i][(int64_t)lane * a.rows] : 0.f;
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    lse2[i] = -INFINITY;
-    if (n[i] > 1) {
-      float mx = -INFINITY;
-      if (lane < n[i]) mx = fmaxf(mx, l0[i]);
-      for (int k = lane + 64; k < n[i]; k += 64) mx = fmaxf(mx, lsep[i][(int64_t)k * a.rows]);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-      float sum = 0.f;
-      if (mx != -INFINITY) {
-        if (lane < n[i]) sum += fast_exp2(l0[i] - mx);
-        for (int k = lane + 64; k < n[i]; k += 64) sum += fast_exp2(lsep[i][(int64_t)k * a.rows] - mx);
-      }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-      lse2[i] = sum > 0.f ? mx + __log2f(sum) : -INFINITY;
-      if (lane == 0 && a.lse != nullptr) {
-        const int m = m0 + r0 + i;
-        const int b = m / a.s_q, s = m - b * a.s_q;
-        a.lse[((int64_t)b * a.heads + h) * a.s_q + s] = lse2[i] * kLn2;
-      }
+  // ---- 2. merge row m0 + wave
+  const int m0 = blockIdx.y * kAbsRows;
+  const int m = m0 + wave;
+  i32x4 merged = i32x4{0, 0, 0, 0};
+  if (m < a.m_rows) {  // uniform
+    const int b = m / a.s_q, s = m - b * a.s_q;
+    const int row = s * a.heads + h;
+    const int base = a.splits[b];
+    const int n = a.splits[b + 1] - base;
+    if (n == 1 || (a.premerged && n > 1)) {  // the row is in `out`, its lse written
+      merged = *(const i32x4_a8*)(a.out + b * a.o_sb + s * a.o_ss + h * a.o_sh + lane * 8);
+    } else if (n > 1) {
+      float acc[8];
+      const float lse2 = merge_row16<DT, true>(a.ws_o, a.ws_scale, a.ws_lse, base, n, a.rows, row, lane, w_sh[wave], acc);
+      merged = i32x4{(int)pack2<DT>(acc[0], acc[1]), (int)pack2<DT>(acc[2], acc[3]), (int)pack2<DT>(acc[4], acc[5]),
+                     (int)pack2<DT>(acc[6], acc[7])};
+      if (lane == 0 && a.lse != nullptr) a.lse[((int64_t)b * a.heads + h) * a.s_q + s] = lse2 * kLn2;
     }
   }
-  float acc[R][8];
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
-  for (int k0 = 0; k0 < nmax; k0 += 64) {
-    const int k = k0 + lane;
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      float w = 0.f;
-      if (n[i] == 1) {
-        w = 1.f;  // fma(1, x, 0) = x: the single-split row as the decode wrote it
-      } else if (k < n[i] && lse2[i] != -INFINITY) {
-        w = fast_exp2((k0 == 0 ? l0[i] : lsep[i][(int64_t)k * a.rows]) - lse2[i]);
-      }
-      w_sh[r0 + i][lane] = w;
-    }
-    __builtin_amdgcn_wave_barrier();
-    const int kn = nmax - k0 < 64 ? nmax - k0 : 64;
-    for (int kb = 0; kb < kn; kb += kPF) {
-      if (k0 + kb > 0) {
-#pragma unroll
-        for (int u = 0; u < kPF; ++u)
-#pragma unroll
-          for (int i = 0; i < R; ++i)
-            if (k0 + kb + u < n[i]) load_row(k0 + kb + u, i, x[u][i], us[u][i]);
-      }
-#pragma unroll
-      for (int u = 0; u < kPF; ++u)
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-          if (k0 + kb + u < n[i]) {
-            const float wk = w_sh[r0 + i][kb + u] * us[u][i];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[i][j] += wk * x[u][i][j];
-          }
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-    *(i32x4*)&a_sh[(r0 + i) * kPitch + lane * 8] =
-        i32x4{(int)pack2<DT>(acc[i][0], acc[i][1]), (int)pack2<DT>(acc[i][2], acc[i][3]),
-              (int)pack2<DT>(acc[i][4], acc[i][5]), (int)pack2<DT>(acc[i][6], acc[i][7])};
-
-  // ---- 3. this wave's B fragments (8 consecutive k of one column n) in one round trip, then
-  //         the 16 x kVDim product
-  const uint16_t* wb0 = a.w_blk + (int64_t)h * kVDim * kDV + (32 * wave + li) * 32 + 8 * g;
-  i32x4 bf[KS][NT];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bf[ks][nt] = *(const i32x4*)(wb0 + (ks * kVDim + 16 * nt) * 32);
+  *(i32x4*)&a_sh[wave * kPitch + lane * 8] = merged;
   __syncthreads();
-  f32x4 c[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) c[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- 3. this wave's v^T tile over its contraction half
+  f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    const i32x4 af = *(const i32x4*)&a_sh[li * kPitch + 32 * ks + 8 * g];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) c[nt] = mfma32<DT>(af, bf[ks][nt], c[nt]);
+    const i32x4 rf = *(const i32x4*)&a_sh[li * kPitch + 32 * (kh * KS + ks) + 8 * g];
+    c = mfma32<DT>(wf[ks], rf, c);
   }
-  // lane (g, li) holds rows 4g .. 4g+3 of column li of each tile
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + 4 * g + r;
-      if (m < a.m_rows) {
-        const float v = c[nt][r];
-        const uint32_t pk = pack2<DT>(v, v);
-        a.v[((int64_t)m * a.heads + h) * kVDim + 32 * wave + 16 * nt + li] = (uint16_t)(pk & 0xFFFF);
-      }
-    }
+  if (kh == 1) c_sh[nt][lane] = c;  // uniform
+  __syncthreads();
+  if (kh == 0) {  // uniform: lane (g, li) holds columns 16 nt + 4g .. +3 of row li
+    c += c_sh[nt][lane];
+    if (m0 + li < a.m_rows)
+      *(i32x2_a4*)(a.v + ((int64_t)(m0 + li) * a.heads + h) * kVDim + 16 * nt + 4 * g) =
+          i32x2{(int)pack2<DT>(c[0], c[1]), (int)pack2<DT>(c[2], c[3])};
+  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3982,9 +3873,9 @@ int mla_combine_absorb(const mla_decode_args* args, const void* w_uv_blk, void* 
   }
   const dim3 grid(kp.heads, (a.m_rows + mla::kAbsRows - 1) / mla::kAbsRows);
   if (args->dtype == MLA_DTYPE_BF16)
-    hipLaunchKernelGGL(mla::mla_combine_absorb_kernel<MLA_DTYPE_BF16>, grid, dim3(256), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(mla::mla_combine_absorb_kernel<MLA_DTYPE_BF16>, grid, dim3(64 * mla::kAbsRows), 0, (hipStream_t)stream, a);
   else
-    hipLaunchKernelGGL(mla::mla_combine_absorb_kernel<MLA_DTYPE_F16>, grid, dim3(256), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(mla::mla_combine_absorb_kernel<MLA_DTYPE_F16>, grid, dim3(64 * mla::kAbsRows), 0, (hipStream_t)stream, a);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MLA_ERR_HIP, std::string("combine-absorb launch failed: ") + hipGetErrorString(e));
   return MLA_OK;

@@ -209,3 +209,25 @@ def test_absorb_long_single_sequence(gpu, H):
     ref_o, _ = R.decode_paged(inp.q, inp.kv_cache, inp.block_table, inp.cache_seqlens, inp.sm_scale, True)
     ref_v = torch.einsum("bshk,hkn->bshn", ref_o, w_uv.float())
     check_close(v, ref_v, V_RTOL * ref_v.abs().max().item(), f"v long H={H}")
+
+
+@pytest.mark.parametrize("B", [15, 17, 32])
+def test_absorb_row_tiles_and_long_merge(gpu, B):
+    """Batches at the edges of the 16-row tiles; the first sequence's merge is longer than one
+    64-split weight window while the batch average stays below the dim-quarter combine's."""
+    H = 16
+    cfg = small_cfg("absorb_tiles", B, 1, H, [6000] + [1 + 7 * i for i in range(B - 1)])
+    inp = make_inputs(cfg, seed=60 + B)
+    w_uv, _ = weights(H, torch.bfloat16, B)
+    d = inp.to("cuda")
+    say(f"absorb row tiles B={B}")
+    sched, splits = get_mla_metadata(d.cache_seqlens, H, 1, num_parts=15 * B + 1, fixed_overhead=0)
+    args = (d.q, d.kv_cache, d.block_table, d.cache_seqlens)
+    v, lse = mla_decode_absorbed(*args, sched, splits, prepare_w_uv(w_uv.cuda()), softmax_scale=inp.sm_scale, causal=True)
+    out, lse2 = flash_mla_with_kvcache(*args, 512, sched, splits, softmax_scale=inp.sm_scale, causal=True)
+    torch.cuda.synchronize()
+    assert int(splits[1]) > 64 and sched.shape[0] < 16 * B
+    ref_o, _ = R.decode_paged(inp.q, inp.kv_cache, inp.block_table, inp.cache_seqlens, inp.sm_scale, True)
+    ref_v = torch.einsum("bshk,hkn->bshn", ref_o, w_uv.float())
+    check_close(v, ref_v, V_RTOL * ref_v.abs().max().item(), f"v row tiles B={B}")
+    _fused_equals_combine(v, lse, out, lse2, w_uv, f"row tiles B={B}")
