@@ -300,6 +300,17 @@ __device__ __forceinline__ void dma16_lane(const void* addr, uint32_t lds_addr) 
       : "v"(addr), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
       : "memory", "m0");
 }
+// The per-lane-address copy with the destination and the address stepped as in dma16_m0.
+template <int LDS_OFF, int GOFF>
+__device__ __forceinline__ void dma16_lane_m0(uint64_t addr, uint32_t lds_base) {
+  static_assert(GOFF >= 0 && GOFF < 4096 && LDS_OFF - GOFF > -65536, "immediate offset range");
+  asm volatile(
+      "s_add_u32 m0, %1, %2\n\t"
+      "global_load_lds_dwordx4 %0, off offset:%3 nt"
+      :
+      : "v"(addr), "s"(lds_base), "i"(LDS_OFF - GOFF), "i"(GOFF)
+      : "memory", "m0", "scc");
+}
 // 4 bytes per lane from a per-lane address, to LDS at lds_addr + 4 * lane (sparse fp8 scales).
 __device__ __forceinline__ void dma4_lane(const void* addr, uint32_t lds_addr) {
   asm volatile(
@@ -1693,7 +1704,17 @@ constexpr int kWidePanel = 16 * 1024;        // tokens 16..31 of a latent stage
 // xcd_hb workgroups (a multiple of 8), xcd_slots = its size / 8; XCD x runs a contiguous block
 // of parts, the xcd_hb head blocks of a part in consecutive slots.  xcd_hb = 0: a (part, head
 // block) grid.  Both are preloaded arguments too: the part index needs them before the record.
-template <int DT, int HT, bool FUSED>
+// SPARSE: the keys of a sequence are the pool tokens its index list names (s_q = 1).  A wave keeps
+// the indices of its own row group (8 of a stage's 32 rows) for kSparseWin stages in LDS, and each
+// lane forms the 64-bit address of its row from them; which of a stage's tokens are keys at all is
+// one word per stage, formed at the segment's start.  The list is requested ahead of the queries, so
+// a segment still starts after two memory round trips (with it after them, three more: 61.7 against
+// 54.5 us).  Main kernel / call against the one-ring kernel: 64 sequences x 128 heads, top 2048,
+// 68.7 -> 54.5 / 73.8 -> 60.2 us; 132 x 64 heads, call 105 -> 76 us; 132 x 48 heads, top 1000, 64 -> 48.
+// (The loads keep the non-temporal hint, 54.5 against 56.0 us: no other workgroup reads the rows.
+// Reading a stage's indices an iteration ahead changed nothing.)
+constexpr int kSparseWin = 24;  // 3 KiB of indices: what the 128-row form's LDS has left
+template <int DT, int HT, bool FUSED, bool SPARSE = false>
 __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restrict__ sched, int xcd_hb, int xcd_slots,
                                                           KParams p) {
   constexpr int NW = 4;
@@ -1714,6 +1735,8 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
   __shared__ float inv_sh[R];   // 1 / row sum of every row, for the epilogue
   // "score above reference" words, one per stage modulo 4 (see the one-ring kernel)
   __shared__ int over_sh[4];
+  __shared__ int32_t idx_sh[SPARSE ? NW : 1][SPARSE ? 8 * kSparseWin : 1];
+  __shared__ uint32_t vmask_sh[SPARSE ? kSparseMaxTopk / kStageTok + 1 : 1];  // bit i: token i of the stage is a key
   uint8_t LDS_AS* const lat = (uint8_t LDS_AS*)lat_raw;
   uint8_t LDS_AS* const rope = (uint8_t LDS_AS*)rope_raw;
   uint8_t LDS_AS* const ptb = (uint8_t LDS_AS*)pt_raw;
@@ -1787,7 +1810,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     // slots are requested back to back, in that order (nothing waits for the length before it
     // is requested last), so the segment starts after two memory round trips (these loads,
     // then its first stage) instead of one per dependent load.
-    const bool paged = p.block_table != nullptr;
+    const bool paged = !SPARSE && p.block_table != nullptr;
 
     int pbase = 0, bt_lane = 0;
     uint32_t pofs_lo = 0, pofs_hi = 0;  // FUSED: byte offset of page pbase + lane in the cache
@@ -1820,6 +1843,53 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       request_page_ids(first);
       finish_page_ids();
     };
+    // SPARSE: the segment's index list, requested first.  Every wave needs the key masks of all
+    // stages (formed together: 64 indices per wave and turn) and the indices of its own row group.
+    constexpr int kMaskPre = 2;  // turns requested here: 512 indices (more spill)
+    constexpr int kWinLoads = 8 * kSparseWin / 64;
+    const int32_t* idx_list = nullptr;
+    int seg_tok = 0;  // indices in the segment
+    int win0 = 0;     // first stage of the wave's index window
+    int iv[SPARSE ? kMaskPre : 1], wv[SPARSE ? kWinLoads : 1];
+    // the wave's indices of stages win0 .. win0 + kSparseWin - 1; a row past the list re-reads the
+    // last one, an index outside the pool reads pool token 0 (both are masked)
+    auto request_window = [&]() __attribute__((always_inline)) {
+      const int ln = fresh_lane();
+#pragma unroll
+      for (int i = 0; i < kWinLoads; ++i) {
+        const int e = 64 * i + ln;
+        const int t = (win0 + (e >> 3)) * kStageTok + 8 * wave + (e & 7);
+        wv[i] = idx_list[t < seg_tok ? t : seg_tok - 1];
+      }
+    };
+    auto store_window = [&]() __attribute__((always_inline)) {
+      const int ln = fresh_lane();
+#pragma unroll
+      for (int i = 0; i < kWinLoads; ++i)
+        idx_sh[wave][64 * i + ln] = wv[i] < 0 || (int64_t)wv[i] >= p.pool_tokens ? 0 : wv[i];
+      wait_lgkm0();
+      asm volatile("" ::: "memory");  // read by other lanes of this wave only
+    };
+    auto load_window = [&](int first) __attribute__((always_inline)) {
+      win0 = first;
+      request_window();
+      store_window();
+    };
+    if constexpr (SPARSE) {
+      const int last_page = (b == end_b) ? end_page : pages_of(p.topk);
+      const int tok0 = page * kPageTokens;
+      const int tok1 = last_page * kPageTokens < p.topk ? last_page * kPageTokens : p.topk;
+      idx_list = p.indices + (int64_t)b * p.idx_stride + tok0;
+      seg_tok = tok1 - tok0;
+      if (seg_tok > 0) {  // uniform
+        request_window();
+#pragma unroll
+        for (int i = 0; i < kMaskPre; ++i) {
+          const int t = 64 * (NW * i + wave) + fresh_lane();
+          iv[i] = idx_list[t < seg_tok ? t : seg_tok - 1];
+        }
+      }
+    }
     // ---- query fragments of this wave's rows (B operand of S^T = K Q^T), resident for the
     // segment; rows past the end re-load the last row (their results are never written).
     // The addresses come from a fresh lane id and an opaque copy of the head count: otherwise
@@ -1850,7 +1920,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     // the length and the sequence's workspace slots (loaded here so that the epilogue does not
     // wait on them); awaiting the length also awaits everything above (vmcnt is in order),
     // which is in flight by then
-    const int l_raw = p.seqlens[b];
+    const int l_raw = SPARSE ? p.topk : p.seqlens[b];
     const int slot0 = p.splits[b];
     const bool single = (p.splits[b + 1] - slot0) == 1;
     const int L = bound_seq_len(p, l_raw, paged);
@@ -1866,6 +1936,27 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     for (int ht = 0; ht < HT; ++ht) lim[ht] = L - (p.causal ? (p.s_q - 1 - qtok[ht]) : 0);
     const int lmin = L - (p.causal ? p.s_q - 1 : 0);  // every row sees tokens < lmin
 
+    if constexpr (SPARSE) {
+      if (nst > 0) {  // uniform
+        // 64 indices, two stages; read after the pass's first barrier
+        auto put_masks = [&](int t0, int v) __attribute__((always_inline)) {
+          const uint64_t m =
+              __builtin_amdgcn_ballot_w64(t0 + fresh_lane() < seg_tok && v >= 0 && (int64_t)v < p.pool_tokens);
+          vmask_sh[t0 / kStageTok] = (uint32_t)m;  // every lane, one value
+          vmask_sh[t0 / kStageTok + 1] = (uint32_t)(m >> 32);
+        };
+#pragma unroll
+        for (int i = 0; i < kMaskPre; ++i)
+          if (64 * (NW * i + wave) < seg_tok) put_masks(64 * (NW * i + wave), iv[i]);  // uniform
+#pragma unroll 1
+        for (int t0 = 64 * (NW * kMaskPre + wave); t0 < seg_tok; t0 += 64 * NW) {
+          const int t = t0 + fresh_lane();
+          put_masks(t0, idx_list[t < seg_tok ? t : seg_tok - 1]);
+        }
+        store_window();
+      }
+    }
+
     f32x4 o[WDT][RT];
     // row sums of this wave's QK rows: l_part over P as rounded for PV (normalises the
     // output), l_exact over the fp32 P (gives the lse)
@@ -1880,6 +1971,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       uint64_t nb, rb;  // latent and rope row bases of the stage (bytes, uniform)
       uint32_t on, orp; // per-lane byte offsets
       uint32_t lat_dst, rope_dst;  // LDS destinations (uniform)
+      uint64_t an, ar;  // SPARSE: the lane's latent and rope addresses
     };
     // A stage past the segment (the loop's last iterations) is still issued, to the ring slot
     // that is free at that point, with every lane reading the segment's last row: the loads
@@ -1888,6 +1980,28 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       const bool real = k < nst;
       const int st = st_begin + (real ? k : nst - 1);
       StageIssue si;
+      si.lat_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+          (int)(uint32_t)(uintptr_t)(lat + (k % kWideLat) * kLatStageBytes + wave * 8 * 1024));
+      si.rope_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+          (int)(uint32_t)(uintptr_t)(rope + (k % kWideRope) * kRopeStageBytes + wave * 1024));
+      if constexpr (SPARSE) {
+        const int ks = real ? k : (nst > 0 ? nst - 1 : 0);
+        if (ks - win0 >= kSparseWin) load_window(ks);  // uniform
+        const int ln = fresh_lane();
+        int v = idx_sh[wave][(ks - win0) * 8 + (ln >> 3)];
+        uint32_t cl = (uint32_t)(((ln & 7) ^ stage_swz(((wave & 1) << 3) | (ln >> 3))) << 4);
+        if (!real) {  // uniform: one line
+          v = __builtin_amdgcn_readfirstlane(v);
+          cl = 0;
+        }
+        const uint32_t pg = (uint32_t)(v >> 6), rw = (uint32_t)(v & 63);
+        si.an = (uint64_t)(uintptr_t)p.kv_nope + cl +
+                2 * ((uint64_t)pg * (uint32_t)p.kv_sp + rw * (uint32_t)kv_st);
+        si.ar = FUSED ? si.an
+                      : (uint64_t)(uintptr_t)p.kv_rope + cl +
+                            2 * ((uint64_t)pg * (uint32_t)p.kr_sp + rw * (uint32_t)kr_st);
+        return si;
+      }
       const int tok = (st & 1) * kStageTok;
       const char* nb;
       const char* rb;
@@ -1922,15 +2036,14 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       const uint32_t cl = real ? (uint32_t)(((lane & 7) ^ stage_swz(((wave & 1) << 3) | (lane >> 3))) << 4) : 0u;
       si.on = (uint32_t)(row * kv_st) * 2 + cl;
       si.orp = FUSED ? si.on : (uint32_t)(row * kr_st) * 2 + cl;
-      si.lat_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
-          (int)(uint32_t)(uintptr_t)(lat + (k % kWideLat) * kLatStageBytes + wave * 8 * 1024));
-      si.rope_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
-          (int)(uint32_t)(uintptr_t)(rope + (k % kWideRope) * kRopeStageBytes + wave * 1024));
       return si;
     };
     auto issue_one = [&](const StageIssue& si, auto jtag) __attribute__((always_inline)) {
       constexpr int j = decltype(jtag)::value;
-      if constexpr (j < 8) dma16_m0<j * 1024, 128 * j>(si.nb, si.on, si.lat_dst);
+      if constexpr (SPARSE) {
+        if constexpr (j < 8) dma16_lane_m0<j * 1024, 128 * j>(si.an, si.lat_dst);
+        else dma16_lane_m0<0, FUSED ? 1024 : 0>(si.ar, si.rope_dst);
+      } else if constexpr (j < 8) dma16_m0<j * 1024, 128 * j>(si.nb, si.on, si.lat_dst);
       else if constexpr (FUSED) dma16_m0<0, 1024>(si.nb, si.on, si.rope_dst);  // rope = latent row + 1024 B
       else dma16_m0<0>(si.rb, si.orp, si.rope_dst);
     };
@@ -1990,7 +2103,11 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       // the first pass uses the page ids loaded in the prologue; a pass after an abort reloads
       // the window the segment starts in.  The compiler's wait for the ids (and for the query
       // fragments, before the first MFMA) counts only the loads issued after them.
-      if (pbase != page) load_page_ids(page);  // uniform
+      if constexpr (SPARSE) {
+        if (win0 != 0) load_window(0);  // uniform
+      } else {
+        if (pbase != page) load_page_ids(page);  // uniform
+      }
       if (0 < nst) issue(0);
       if (1 < nst) issue(1);
 
@@ -2073,9 +2190,21 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
 
       // mask tokens past each row's limit (uniform branch: the last stages only), then each
       // lane's largest scaled score per row tile
-      auto mask_max = [&](int k, f32x4 (&acc)[HT][2], float (&lmx)[HT]) __attribute__((always_inline)) {
+      // vm (SPARSE): the stage's key mask; the list's tail is masked by it too
+      auto mask_max = [&](int k, f32x4 (&acc)[HT][2], float (&lmx)[HT], uint32_t vm) __attribute__((always_inline)) {
         const int st = st_begin + k;
-        if (st * kStageTok + kStageTok > lmin) {
+        if constexpr (SPARSE) {
+          if (vm != ~0u) {  // uniform
+            const uint32_t mg = vm >> (4 * (fresh_lane() >> 4));
+#pragma unroll
+            for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+              for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  if (!((mg >> (16 * tt + r)) & 1u)) acc[ht][tt][r] = -INFINITY;
+          }
+        } else if (st * kStageTok + kStageTok > lmin) {
 #pragma unroll
           for (int ht = 0; ht < HT; ++ht) {
             int rel = lim[ht] - st * kStageTok - 4 * g;
@@ -2127,7 +2256,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       // `over` test), so the MFMA pipe goes from QK to PV without a gap; at 64 rows that placement
       // makes the register allocator spill, and mask_late_in_pv is false.
       auto pv_softmax = [&](int kp, f32x4 (&acc)[HT][2], const i32x4 (&va)[WDT], const i32x4 (&bq_in)[2],
-                            const StageIssue& si, const LaneOffsets& lo,
+                            const StageIssue& si, const LaneOffsets& lo, uint32_t vm,
                             bool& over) __attribute__((always_inline)) {
         uint8_t LDS_AS* pw = ptb + ((kp + 1) & 1) * kPBytes + lo.pt;
         float mu[HT];
@@ -2162,7 +2291,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
             // readable (the documented need is at most 19 wait states)
             qk_settle_after_mfmas(acc);
             float lmx[HT];
-            mask_max(kp + 1, acc, lmx);
+            mask_max(kp + 1, acc, lmx, vm);
             if constexpr (MODE == kPassFirstStageRef) {
 #pragma unroll
               for (int ht = 0; ht < HT; ++ht) over |= lmx[ht] > m_ref[ht] + kTau;
@@ -2201,7 +2330,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         i32x4 va_unused[WDT], bq_unused[2];
         qk(0, acc, lo, StageIssue{}, std::false_type{}, false, va_unused, bq_unused);
         float lmx[HT];
-        mask_max(0, acc, lmx);
+        mask_max(0, acc, lmx, SPARSE ? (uint32_t)__builtin_amdgcn_readfirstlane((int)vmask_sh[0]) : ~0u);
         if constexpr (MODE == kPassRowMax) {
 #pragma unroll
           for (int ht = 0; ht < HT; ++ht) m_ref[ht] = fmaxf(m_ref[ht], lmx[ht]);
@@ -2237,6 +2366,8 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
           flag_word = over_sh[(k - 1) & 3];
           if (k >= 3 && wave == 0) over_sh[(k - 2) & 3] = 0;
         }
+        uint32_t vm = ~0u;
+        if constexpr (SPARSE) vm = (uint32_t)__builtin_amdgcn_readfirstlane((int)vmask_sh[k]);
         if constexpr (!kPrepEarly) si = prepare(k + 2);  // past the segment: dummy loads
         // 64-row form: from a fresh lane id per iteration (kept live across the loop they
         // spill); 128-row form: once per pass (no spill there, 27 fewer VALU per stage)
@@ -2276,7 +2407,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         bool over = false;
         if constexpr (!kPV || !kMaskLate) {
           float lmx[HT];
-          mask_max(k, acc, lmx);
+          mask_max(k, acc, lmx, vm);
           if constexpr (MODE == kPassRowMax) {
 #pragma unroll
             for (int ht = 0; ht < HT; ++ht) m_ref[ht] = fmaxf(m_ref[ht], lmx[ht]);
@@ -2286,7 +2417,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
           }
         }
         if constexpr (kPV) {
-          pv_softmax(k - 1, acc, va, bq, si, lo, over);
+          pv_softmax(k - 1, acc, va, bq, si, lo, vm, over);
         } else {
 #pragma unroll
           for (int j = 4; j < 9; ++j) issue_j(si, j);
@@ -3471,8 +3602,8 @@ hipError_t launch_main(const mla::KParams& kp, int head_blocks, hipStream_t st) 
   return hipGetLastError();
 }
 
-// The 64- and 128-row dense decodes run the wide kernel (PV split by dims across the waves)
-// unless MLA_WIDE=0 selects the one-ring four-wave kernel (kept for the fp8 and sparse paths).
+// The 64- and 128-row decodes over a 16-bit cache run the wide kernel (PV split by dims across the
+// waves) unless MLA_WIDE=0 selects the one-ring four-wave kernel (which the fp8 cache runs).
 bool wide_enabled() {
   static std::once_flag once;
   static bool on = true;
@@ -3483,28 +3614,28 @@ bool wide_enabled() {
   return on;
 }
 
-template <int DT, int HT, bool FUSED>
+template <int DT, int HT, bool FUSED, bool SPARSE>
 void launch_wide_form(const mla::KParams& kp, int head_blocks, hipStream_t st) {
   const int wgs = kp.num_parts * head_blocks;
   if (wgs % 8 == 0) {  // XCD-blocked 1-D grid (see the kernel)
-    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED>), dim3(wgs), dim3(256), 0, st, kp.sched, head_blocks, wgs / 8,
-                       kp);
+    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED, SPARSE>), dim3(wgs), dim3(256), 0, st, kp.sched, head_blocks,
+                       wgs / 8, kp);
   } else {
-    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED>), dim3(kp.num_parts, head_blocks), dim3(256), 0, st, kp.sched,
-                       0, 0, kp);
+    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED, SPARSE>), dim3(kp.num_parts, head_blocks), dim3(256), 0, st,
+                       kp.sched, 0, 0, kp);
   }
 }
 
 // The fused-rope form for the 128-row kernel only (the 64-row one measured 2% slower with it).
-template <int DT, int HT>
+template <int DT, int HT, bool SPARSE = false>
 hipError_t launch_wide(const mla::KParams& kp, int head_blocks, hipStream_t st) {
   if constexpr (HT == 2) {
     if (kp.rope_fused) {
-      launch_wide_form<DT, HT, true>(kp, head_blocks, st);
+      launch_wide_form<DT, HT, true, SPARSE>(kp, head_blocks, st);
       return hipGetLastError();
     }
   }
-  launch_wide_form<DT, HT, false>(kp, head_blocks, st);
+  launch_wide_form<DT, HT, false, SPARSE>(kp, head_blocks, st);
   return hipGetLastError();
 }
 
@@ -3521,6 +3652,8 @@ hipError_t launch_main_dt(const Variant& v, const mla::KParams& kp, int head_blo
     }
     if (v.ws) return launch_main<DT, 4, 1, 1, true, false, true>(kp, head_blocks, st);
     if (v.nw == 1) return launch_main<DT, 1, 2, 1, false, false, true>(kp, head_blocks, st);
+    if (wide_enabled())
+      return v.ht == 1 ? launch_wide<DT, 1, true>(kp, head_blocks, st) : launch_wide<DT, 2, true>(kp, head_blocks, st);
     if (v.ht == 1) return launch_main<DT, 4, 1, 4, false, false, true>(kp, head_blocks, st);
     return launch_main<DT, 4, 2, 3, false, false, true>(kp, head_blocks, st);
   }
@@ -3653,8 +3786,8 @@ mla::KParams make_params(const mla_decode_args* a) {
   // one cache tensor: the rope half starts 512 elements into each latent row, same strides
   k.rope_fused = (const uint16_t*)a->kv_rope == (const uint16_t*)a->kv_nope + mla::kDV &&
                  a->kv_rope_stride_tok == a->kv_stride_tok &&
-                 (a->block_table ? a->kv_rope_stride_page == a->kv_stride_page
-                                 : a->kv_rope_stride_batch == a->kv_stride_batch) &&
+                 (a->block_table || a->indices ? a->kv_rope_stride_page == a->kv_stride_page
+                                               : a->kv_rope_stride_batch == a->kv_stride_batch) &&
                  a->kv_format == MLA_KV_NATIVE;
   return k;
 }

@@ -112,3 +112,37 @@ def test_sparse_fp8_cache(gpu, H):
     o16, l16 = run_sparse(q, deq.to(torch.bfloat16), idx)
     assert (out.float() - o16.float()).abs().max().item() <= 4e-3
     assert (lse - l16).abs().max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("H,dtype,views", [(64, torch.float16, False), (64, torch.bfloat16, True), (128, torch.bfloat16, False),
+                                           (128, torch.bfloat16, True), (150, torch.float16, False)])
+@pytest.mark.parametrize("topk,forced", [(2048, 1), (1600, 2), (769, 1), (768, 1), (5, 1)])
+def test_sparse_wide_index_windows(gpu, H, dtype, views, topk, forced):
+    """More than 32 heads: lists longer than the kernel's index window (768 tokens), lists ending
+    at its edge, a first stage without keys, a list without keys, and scores that make a segment
+    be redone after its window has moved; one cache tensor or two halves of other strides."""
+    q, kv, idx = sparse_case(4, H, topk, nb=40, seed=H + topk, dtype=dtype)
+    idx[0, 0, :33] = -1
+    idx[1] = -1
+    # a key far above every other score of sequence 2's first head, through its rope dims: a
+    # score of ~ 64 * 30 / 24 = 80, past the reference margins (64 / 15 log2 units).  Its V row is
+    # that head's output, so it is kept below 2, where half a bf16 ulp is at most 2^-8 = 0.004 of the
+    # 0.01 bar (a first form set the row to 4 q: |out| up to 13, half an ulp 0.03)
+    kv[39, 63, 0, 512:] = q[2, 0, 0, 512:] * 30
+    kv[39, 63, 0, :512] *= 0.25
+    idx[2, 0, :-1] = idx[2, 0, :-1].clamp(max=39 * 64 + 62)
+    idx[2, 0, -1] = 39 * 64 + 63
+    say(f"sparse wide H={H} {dtype} views={views} topk={topk} forced={forced}")
+    ref_o, ref_l = R.decode_sparse(q, kv, idx, 576 ** -0.5)
+    dummy = torch.zeros(4, dtype=torch.int32, device="cuda")
+    sched, splits = get_mla_metadata(dummy, H, 1, topk=topk, forced_splits=forced)
+    cache = kv.cuda()
+    if views:  # the rope half in a tensor of its own, the latent rows 520 elements apart
+        lat = torch.zeros(40, 64, 1, 520, dtype=dtype, device="cuda")
+        lat[..., :512] = cache[..., :512]
+        cache = (lat[..., :512], cache[..., 512:].contiguous())
+    out, lse = flash_mla_with_kvcache(q.cuda(), cache, None, None, 512, sched, splits, softmax_scale=576 ** -0.5,
+                                      indices=idx.cuda())
+    torch.cuda.synchronize()
+    assert torch.all(out[1] == 0) and torch.all(lse[1] == float("-inf"))
+    assert_parity(out, lse, ref_o, ref_l, f"sparse wide H={H} topk={topk}")
