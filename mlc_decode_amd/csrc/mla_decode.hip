@@ -300,6 +300,15 @@ __device__ __forceinline__ void dma16_lane(const void* addr, uint32_t lds_addr) 
       : "v"(addr), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
       : "memory", "m0");
 }
+// 4 bytes per lane (SGPR base + 32-bit lane offset), to LDS at lds_base + 4 * lane.
+__device__ __forceinline__ void dma4_m0(uint64_t sbase, uint32_t voff, uint32_t lds_base) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "global_load_lds_dword %0, %1"
+      :
+      : "v"(voff), "s"(sbase), "s"(lds_base)
+      : "memory", "m0");
+}
 // The per-lane-address copy with the destination and the address stepped as in dma16_m0.
 template <int LDS_OFF, int GOFF>
 __device__ __forceinline__ void dma16_lane_m0(uint64_t addr, uint32_t lds_base) {
@@ -1714,9 +1723,23 @@ constexpr int kWidePanel = 16 * 1024;        // tokens 16..31 of a latent stage
 // (The loads keep the non-temporal hint, 54.5 against 56.0 us: no other workgroup reads the rows.
 // Reading a stage's indices an iteration ahead changed nothing.)
 constexpr int kSparseWin = 24;  // 3 KiB of indices: what the 128-row form's LDS has left
-template <int DT, int HT, bool FUSED, bool SPARSE = false>
+// KV8 (fp8 latent cache, paged): a wave loads the codes and scales of its own row group into raw
+// slots that only it reads, and turns them into the bf16 stage that all waves read, between the
+// MFMAs of PV (where LDS is least busy): in iteration k it dequantises stage k + 1 into the bf16
+// slot that stage k - 2 left, then refills the raw slot with stage k + 3.  So QK and PV are the
+// 16-bit kernel's, one barrier a stage serves both, and every code is converted once per
+// workgroup.  The one-ring kernel dequantises between two barriers, with no MFMA to hide it.  Main
+// kernel / call, 64 sequences x 128 heads x 4096 tokens: 112 -> 90 / 114.8 -> 93.8 us (86 over the
+// bf16 cache); calls: 32 x 16384, 2 x 128 rows 380 -> 304 us, 132 skewed x 64 heads 66.5 -> 59.2.
+// At 128 rows it fits the registers only without the late masking below: with it the compiler
+// spills a query fragment, whose reload waits for every load in flight (106 us).
+constexpr int kRaw8Bytes = 16 * 1024;  // codes of one stage
+template <int DT, int HT, bool FUSED, bool SPARSE = false, bool KV8 = false>
 __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restrict__ sched, int xcd_hb, int xcd_slots,
                                                           KParams p) {
+  static_assert(!KV8 || (DT == MLA_DTYPE_BF16 && !FUSED && !SPARSE), "the fp8 form: bf16 queries, paged");
+  constexpr int kLat = KV8 ? 3 : kWideLat;  // bf16 stages resident (KV8: and two raw stages behind them)
+  constexpr int kLead = KV8 ? 3 : 2;        // iteration k issues stage k + kLead
   constexpr int NW = 4;
   constexpr int RT = NW * HT;        // 16-row tiles per workgroup
   constexpr int R = 16 * RT;         // rows per workgroup
@@ -1724,10 +1747,11 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
   constexpr int DK = 4;              // LDS prefetch depth of the QK A fragments
   // Three placements in the stage loop that pay at 128 rows per workgroup and cost at 64 (C2 main
   // kernel 87.7 -> 86.5 us with all three; C5 50.5 -> 49.1 us with none of them at 64 rows):
-  constexpr bool kMaskLate = HT == 2;   // QK results first read inside PV's first step
+  constexpr bool kMaskLate = HT == 2 && !KV8;   // QK results first read inside PV's first step
   constexpr bool kPtEarly = HT == 2;    // PV's first P^T fragments read at the end of QK
   constexpr bool kPrepEarly = HT == 2;  // stage k + 2's loads prepared at the end of iteration k - 1
   constexpr float kTau = ref_tau<DT>();
+  constexpr float kMinRef = -3.4028234664e38f;
   constexpr int kPBytes = RT * 1024;
   __shared__ __attribute__((aligned(1024))) uint8_t lat_raw[kWideLat * kLatStageBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t rope_raw[kWideRope * kRopeStageBytes];
@@ -1736,6 +1760,9 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
   // "score above reference" words, one per stage modulo 4 (see the one-ring kernel)
   __shared__ int over_sh[4];
   __shared__ int32_t idx_sh[SPARSE ? NW : 1][SPARSE ? 8 * kSparseWin : 1];
+  // KV8: the scales [row][128-dim block] of each wave's row group, two stages (the upper half of a
+  // wave's 256 bytes repeats the lower)
+  __shared__ __attribute__((aligned(16))) float scale_sh[KV8 ? 2 : 1][KV8 ? NW : 1][KV8 ? 64 : 1];
   __shared__ uint32_t vmask_sh[SPARSE ? kSparseMaxTopk / kStageTok + 1 : 1];  // bit i: token i of the stage is a key
   uint8_t LDS_AS* const lat = (uint8_t LDS_AS*)lat_raw;
   uint8_t LDS_AS* const rope = (uint8_t LDS_AS*)rope_raw;
@@ -1784,6 +1811,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
   // (v_lane ^ 32*d4) + 1024*s.  Wave w's segments are 2w and 2w + 1.
   struct LaneOffsets {
     int kl0, kl1, kr0, kr1, v, pt;
+    int dq;  // KV8: the lane's codes in a raw block (see dequant)
   };
   // The chunks 2g and 2g + 1 of a row differ in bit 0, which the swizzle leaves in place, so
   // kl1 = kl0 ^ 16 and kr1 = kr0 ^ 16; kr0 is kl0 with its row-group bit (8 KiB) moved to 1 KiB.
@@ -1798,6 +1826,11 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     o.kr1 = o.kr0 ^ 16;
     o.v = (r >> 3) * 8192 + ((r & 7) << 7) + ((((ll >> 1) & 1) ^ stage_swz(r)) << 4) + ((ll & 1) << 3) + 2048 * wave;
     o.pt = 16 * ln;
+    // lane (r8, i) = (ln / 8, ln % 8) converts chunk c8 = i ^ swz of row 8 * wave + r8 in every 64-dim
+    // segment: 8 codes, half c8 % 2 of 16-byte chunk c8 / 2 (+ 4 in odd segments); the load leaves
+    // 16-byte chunk j of a row at slot j ^ 4 * (r8 / 2 % 2), so four rows' reads cover all banks
+    const int c8 = (ln & 7) ^ stage_swz(((wave & 1) << 3) | (ln >> 3));
+    o.dq = ((ln >> 3) << 7) + ((c8 >> 1) << 4) + ((c8 & 1) << 3) + (((ln >> 4) & 1) << 6);
     return o;
   };
 
@@ -1810,7 +1843,9 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     // slots are requested back to back, in that order (nothing waits for the length before it
     // is requested last), so the segment starts after two memory round trips (these loads,
     // then its first stage) instead of one per dependent load.
-    const bool paged = !SPARSE && p.block_table != nullptr;
+    // (a constant for KV8: a test of it around the page-id load and another around its use leave the
+    // compiler a path that waits for the load, and with it for every stage load, in each iteration)
+    const bool paged = KV8 || (!SPARSE && p.block_table != nullptr);
 
     int pbase = 0, bt_lane = 0;
     uint32_t pofs_lo = 0, pofs_hi = 0;  // FUSED: byte offset of page pbase + lane in the cache
@@ -1960,6 +1995,8 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     f32x4 o[WDT][RT];
     // row sums of this wave's QK rows: l_part over P as rounded for PV (normalises the
     // output), l_exact over the fp32 P (gives the lse)
+    // The reference max is kept finite (at least -FLT_MAX): a row without a key so far then needs no
+    // case of its own, since 2^(-inf - m) is 0 and any finite score lies more than tau above.
     float m_ref[HT], l_part[HT], l_exact[HT];
     // The loads of one stage: wave w fetches row group w, 8 latent blocks and 1 rope block (one
     // global_load_lds_dwordx4 each, eight lanes per 128-byte line).  `prepare` does the scalar
@@ -1972,11 +2009,25 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       uint32_t on, orp; // per-lane byte offsets
       uint32_t lat_dst, rope_dst;  // LDS destinations (uniform)
       uint64_t an, ar;  // SPARSE: the lane's latent and rope addresses
+      // KV8: scale base and offsets, raw slot, and the rope base of this stage (issued an iteration
+      // after its codes, from the next record's rb / orp)
+      uint64_t sb, rbn;
+      uint32_t osc, sc_dst;
     };
     // A stage past the segment (the loop's last iterations) is still issued, to the ring slot
     // that is free at that point, with every lane reading the segment's last row: the loads
     // cost a cache line, and the wait counts stay the same in every iteration.
-    auto prepare = [&](int k) __attribute__((always_inline)) {
+    auto lane8 = [&](int last_row, bool real, StageIssue& si) __attribute__((always_inline)) {
+      const int ln = fresh_lane();
+      int row = 8 * wave + (ln >> 3), srow = 8 * wave + ((ln >> 2) & 7);
+      row = row < last_row && real ? row : last_row;
+      srow = srow < last_row && real ? srow : last_row;
+      si.on = (uint32_t)(row * kv_st) + (real ? (uint32_t)(((ln & 7) ^ ((ln >> 4 & 1) << 2)) << 4) : 0u);
+      si.osc = (uint32_t)(srow + (ln & 3) * (int)p.ks_sb) * 4;
+    };
+    // KV8: prev is the record of stage k - 1, whose rope goes out with stage k's codes and whose lane
+    // offsets stage k keeps
+    auto prepare = [&](int k, const StageIssue& prev = StageIssue{}) __attribute__((always_inline)) {
       const bool real = k < nst;
       const int st = st_begin + (real ? k : nst - 1);
       StageIssue si;
@@ -1984,6 +2035,38 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
           (int)(uint32_t)(uintptr_t)(lat + (k % kWideLat) * kLatStageBytes + wave * 8 * 1024));
       si.rope_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
           (int)(uint32_t)(uintptr_t)(rope + (k % kWideRope) * kRopeStageBytes + wave * 1024));
+      const auto uni64 = [](const char* q) {
+        const uint64_t v = (uint64_t)(uintptr_t)q;
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32) |
+               (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+      };
+      if constexpr (KV8) {
+        const int pidx = st >> 1;
+        if (pidx - pbase >= 64) load_page_ids(pidx);  // uniform
+        const uint32_t pg = (uint32_t)__builtin_amdgcn_readlane(bt_lane, pidx - pbase);
+        const int tok = (st & 1) * kStageTok;
+        si.nb = uni64((const char*)p.kv_nope + ((uint64_t)pg * (uint32_t)p.kv_sp + (uint32_t)(tok * kv_st)));
+        si.rbn = uni64((const char*)p.kv_rope + ((uint64_t)pg * (uint32_t)p.kr_sp + (uint32_t)(tok * kr_st)) * 2);
+        si.sb = uni64((const char*)(p.kv_scale + ((int64_t)pg * p.ks_sp + tok)));
+        // the lane's offsets are those of a whole stage up to the sequence's last one (rows past its
+        // end re-read its last row); past the segment every lane reads one line.  The rope rows need
+        // neither: a page holds 64 of them, and what they add to masked scores is dropped.
+        si.on = prev.on;
+        si.osc = prev.osc;
+        if (L - st * kStageTok < kStageTok || !real) {  // uniform; so is every later stage's
+          const int rows = L - st * kStageTok;
+          lane8((rows < kStageTok ? rows : kStageTok) - 1, real, si);
+        }
+        si.rb = prev.rbn;
+        si.orp = prev.orp;
+        si.lat_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(lat + kLat * kLatStageBytes + (k & 1) * kRaw8Bytes + wave * (kRaw8Bytes / NW)));
+        si.rope_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(rope + ((k + kWideRope - 1) % kWideRope) * kRopeStageBytes + wave * 1024));
+        si.sc_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(float LDS_AS*)&scale_sh[k & 1][wave][0]);
+        return si;
+      }
       if constexpr (SPARSE) {
         const int ks = real ? k : (nst > 0 ? nst - 1 : 0);
         if (ks - win0 >= kSparseWin) load_window(ks);  // uniform
@@ -2022,11 +2105,6 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         nb = (const char*)(p.kv_nope + ((int64_t)b * p.kv_sb + (int64_t)st * kStageTok * kv_st));
         rb = (const char*)(p.kv_rope + ((int64_t)b * p.kr_sb + (int64_t)st * kStageTok * kr_st));
       }
-      const auto uni64 = [](const char* q) {
-        const uint64_t v = (uint64_t)(uintptr_t)q;
-        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32) |
-               (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-      };
       si.nb = uni64(nb);
       si.rb = FUSED ? si.nb : uni64(rb);
       const int left = L - st * kStageTok;
@@ -2040,7 +2118,11 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     };
     auto issue_one = [&](const StageIssue& si, auto jtag) __attribute__((always_inline)) {
       constexpr int j = decltype(jtag)::value;
-      if constexpr (SPARSE) {
+      if constexpr (KV8) {  // 0: the previous stage's rope; 1 .. 4: codes; 5: scales
+        if constexpr (j == 0) dma16_m0<0>(si.rb, si.orp, si.rope_dst);
+        else if constexpr (j < 5) dma16_m0<(j - 1) * 1024, 128 * (j - 1)>(si.nb, si.on, si.lat_dst);
+        else dma4_m0(si.sb, si.osc, si.sc_dst);
+      } else if constexpr (SPARSE) {
         if constexpr (j < 8) dma16_lane_m0<j * 1024, 128 * j>(si.an, si.lat_dst);
         else dma16_lane_m0<0, FUSED ? 1024 : 0>(si.ar, si.rope_dst);
       } else if constexpr (j < 8) dma16_m0<j * 1024, 128 * j>(si.nb, si.on, si.lat_dst);
@@ -2074,6 +2156,39 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       issue_one(si, std::integral_constant<int, 8>{});
     };
 
+    // KV8: stage k's codes of this wave's row group (raw slot k % 2) into its bf16 stage, one 64-dim
+    // segment sg at a time: 8 codes per lane, written lane-linearly into block 8 * wave + sg
+    auto dq_read = [&](int k, const LaneOffsets& lo, int sg) __attribute__((always_inline)) {
+      const uint8_t LDS_AS* a = lat + kLat * kLatStageBytes + (k & 1) * kRaw8Bytes + wave * (kRaw8Bytes / NW);
+      return *(const i32x2 LDS_AS*)(a + ((sg & 1) ? lo.dq ^ 64 : lo.dq) + (sg >> 1) * 1024);
+    };
+    auto dq_scale = [&](int k) __attribute__((always_inline)) {
+      return *(const f32x4 LDS_AS*)((const uint8_t LDS_AS*)(const float LDS_AS*)&scale_sh[KV8 ? k & 1 : 0][KV8 ? wave : 0][0] +
+                                    ((fresh_lane() >> 3) << 4));
+    };
+    auto dq_write = [&](int k, const LaneOffsets& lo, int sg, i32x2 raw, float sc) __attribute__((always_inline)) {
+      *(i32x4 LDS_AS*)(lat + (k % kLat) * kLatStageBytes + (8 * wave + sg) * 1024 + lo.pt) = cvt_fp8x8(raw, sc);
+    };
+    // a whole stage; every read of the raw slot has returned when it ends
+    auto dequant = [&](int k) __attribute__((always_inline)) {
+      const LaneOffsets lo = lane_offsets(fresh_lane());
+      f32x4 sc = dq_scale(k);
+      i32x2 raw[8];
+#pragma unroll
+      for (int sg = 0; sg < 8; ++sg) raw[sg] = dq_read(k, lo, sg);
+#pragma unroll
+      for (int sg = 0; sg < 8; ++sg) dq_write(k, lo, sg, raw[sg], sc[sg >> 1]);
+      wait_lgkm0();
+      asm volatile("" ::: "memory");
+    };
+    auto issue_codes = [&](const StageIssue& si) __attribute__((always_inline)) {
+      issue_one(si, std::integral_constant<int, 1>{});
+      issue_one(si, std::integral_constant<int, 2>{});
+      issue_one(si, std::integral_constant<int, 3>{});
+      issue_one(si, std::integral_constant<int, 4>{});
+      issue_one(si, std::integral_constant<int, 5>{});
+    };
+
     // One pass over the segment's stages; returns true (uniformly) when a first-stage-reference
     // pass saw a score above its reference by more than tau.
     //
@@ -2095,7 +2210,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       }
       if constexpr (MODE != kPassFixedRef) {
 #pragma unroll
-        for (int ht = 0; ht < HT; ++ht) m_ref[ht] = -INFINITY;
+        for (int ht = 0; ht < HT; ++ht) m_ref[ht] = kMinRef;
       }
       if constexpr (MODE == kPassFirstStageRef) {
         if (wave == 0) over_sh[lq & 3] = 0;  // uniform branch; ordered by the first barrier
@@ -2108,8 +2223,32 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       } else {
         if (pbase != page) load_page_ids(page);  // uniform
       }
-      if (0 < nst) issue(0);
-      if (1 < nst) issue(1);
+      StageIssue si;
+      if constexpr (KV8) {
+        si = StageIssue{};
+        lane8(kStageTok - 1, true, si);
+        const int ln = fresh_lane();
+        si.orp = (uint32_t)((8 * wave + (ln >> 3)) * kr_st) * 2 +
+                 (uint32_t)(((ln & 7) ^ stage_swz(((wave & 1) << 3) | (ln >> 3))) << 4);
+        // stages 0 and 1 whole (a stage past the segment as a dummy, see prepare), stage 0
+        // dequantised, then stage 2's codes in its raw slot
+        if (0 < nst) {
+          const StageIssue s0 = prepare(0, si), s1 = prepare(1, s0);
+          issue_codes(s0);
+          issue_one(s1, std::integral_constant<int, 0>{});  // rope of stage 0
+          issue_codes(s1);
+          const StageIssue s2 = prepare(2, s1);
+          issue_one(s2, std::integral_constant<int, 0>{});  // rope of stage 1
+          wait_vmcnt<6>();
+          asm volatile("" ::: "memory");
+          dequant(0);
+          issue_codes(s2);
+          si = s2;
+        }
+      } else {
+        if (0 < nst) issue(0);
+        if (1 < nst) issue(1);
+      }
 
       // V^T fragment t (t = 2*d4 + sl: segment 2w + sl, tile d4 in it) of stage kp
       auto v_frag = [&](const uint8_t LDS_AS* vb, int t) __attribute__((always_inline)) {
@@ -2123,7 +2262,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         return i32x4{lo2.x, lo2.y, hi2.x, hi2.y};
       };
       auto v_base = [&](int kp, const LaneOffsets& lo) __attribute__((always_inline)) {
-        const uint8_t LDS_AS* vb = lat + (kp % kWideLat) * kLatStageBytes + lo.v;
+        const uint8_t LDS_AS* vb = lat + (kp % kLat) * kLatStageBytes + lo.v;
         asm volatile("" : "+v"(vb));
         return vb;
       };
@@ -2142,7 +2281,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       // issues eight MFMAs before the softmax reads them (see pv_softmax).
       auto qk = [&](int k, f32x4 (&acc)[HT][2], const LaneOffsets& lo, const StageIssue& si, auto issue_tag,
                     bool vt, i32x4 (&va)[WDT], i32x4 (&bq)[2]) __attribute__((always_inline)) {
-        const uint8_t LDS_AS* lb = lat + (k % kWideLat) * kLatStageBytes;
+        const uint8_t LDS_AS* lb = lat + (k % kLat) * kLatStageBytes;
         const uint8_t LDS_AS* rbs = rope + (k % kWideRope) * kRopeStageBytes;
         const uint8_t LDS_AS* kb0 = lb + lo.kl0;
         const uint8_t LDS_AS* kb1 = lb + lo.kl1;
@@ -2172,7 +2311,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
               mfma_qk<DT>(acc[ht][n & 1], a, qf[ht][n >> 1]);
           }
           if constexpr (decltype(issue_tag)::value) {
-            if ((n & 7) == 4) issue_j(si, n >> 3);  // loads 0..3
+            if ((n & 7) == 4 && (!KV8 || n == 4)) issue_j(si, n >> 3);  // loads 0..3 (KV8: 0)
           }
           if (n >= 2 * kKSteps - WDT && vt) va[n - (2 * kKSteps - WDT)] = v_frag(vb, n - (2 * kKSteps - WDT));
           if (kPtEarly && n >= 2 * kKSteps - 2 && vt) bq[n - (2 * kKSteps - 2)] = pt_frag(k - 1, lo, n - (2 * kKSteps - 2));
@@ -2231,12 +2370,11 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         uint8_t LDS_AS* pw = ptb + (k & 1) * kPBytes + lane * 16;
 #pragma unroll
         for (int ht = 0; ht < HT; ++ht) {
-          const float mu = m_ref[ht] == -INFINITY ? 0.f : m_ref[ht];
           float pv[2][4];
 #pragma unroll
           for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pv[tt][r] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - mu);
+            for (int r = 0; r < 4; ++r) pv[tt][r] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - m_ref[ht]);
           const i32x4 pb = i32x4{(int)pack2<DT>(pv[0][0], pv[0][1]), (int)pack2<DT>(pv[0][2], pv[0][3]),
                                  (int)pack2<DT>(pv[1][0], pv[1][1]), (int)pack2<DT>(pv[1][2], pv[1][3])};
           l_part[ht] = packed_sum<DT>(pb, l_part[ht]);
@@ -2259,15 +2397,12 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
                             const StageIssue& si, const LaneOffsets& lo, uint32_t vm,
                             bool& over) __attribute__((always_inline)) {
         uint8_t LDS_AS* pw = ptb + ((kp + 1) & 1) * kPBytes + lo.pt;
-        float mu[HT];
-#pragma unroll
-        for (int ht = 0; ht < HT; ++ht) mu[ht] = m_ref[ht] == -INFINITY ? 0.f : m_ref[ht];
         float pvv[HT][8];
         // softmax element e of the 8 * HT this lane owns: row tile e / 8, token tile (e / 4) % 2,
         // token 4g + e % 4 of it
         auto p_elem = [&](int e) __attribute__((always_inline)) {
           const int ht = e >> 3, tt = (e >> 2) & 1, r = e & 3;
-          pvv[ht][e & 7] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - mu[ht]);
+          pvv[ht][e & 7] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - m_ref[ht]);
         };
         auto p_finish = [&](int ht) __attribute__((always_inline)) {
           const float* v = pvv[ht];
@@ -2280,6 +2415,21 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         constexpr int kPer = (8 * HT + RT - 1) / RT;  // P elements per step: 2
         i32x4 bq[2] = {bq_in[0], bq_in[1]};
         i32x4 b_last = bq[0];
+        // KV8: stage kp + 2, eight segments over the steps, two reads ahead
+        // (pairs of segments 1 KiB apart: one LDS instruction), in the order 0 2 1 3 4 6 5 7
+        constexpr int kSegs = 8 / RT;
+        const auto seg8 = [](int i) { return (i & 4) | ((i & 1) << 1) | ((i >> 1) & 1); };
+        f32x4 sc8;
+        i32x2 raw8[4];
+        auto read_pair = [&](int i) __attribute__((always_inline)) {
+          raw8[i & 3] = dq_read(kp + 2, lo, seg8(i));
+          raw8[(i & 3) + 1] = dq_read(kp + 2, lo, seg8(i + 1));
+        };
+        if constexpr (KV8) {
+          sc8 = dq_scale(kp + 2);
+          read_pair(0);
+          read_pair(2);
+        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           const i32x4 bcur = bq[rt & 1];
@@ -2305,10 +2455,28 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
               if ((e & 7) == 7) p_finish(e >> 3);
             }
           }
-          // loads 4..8 after steps (2i + 1) * RT / 10
+          if constexpr (KV8) {
 #pragma unroll
-          for (int i = 0; i < 5; ++i)
-            if (rt == (2 * i + 1) * RT / 10) issue_j(si, 4 + i);
+            for (int i = rt * kSegs; i < (rt + 1) * kSegs; ++i) {
+              dq_write(kp + 2, lo, seg8(i), raw8[i & 3], sc8[seg8(i) >> 1]);
+              if ((i & 1) == 1 && i + 3 < 8) read_pair(i + 3);
+              // the raw blocks of segments 0 .. 3 are refilled once the reads of 4 .. 7 are out and
+              // their own have returned, the others at the end
+              if (i == 4) issue_j(si, 1);
+              if (i == 5) issue_j(si, 2);
+              if (i == 7) {
+                asm volatile("" : "+v"(sc8));
+                issue_j(si, 3);
+                issue_j(si, 4);
+                issue_j(si, 5);
+              }
+            }
+          } else {
+            // loads 4..8 after steps (2i + 1) * RT / 10
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+              if (rt == (2 * i + 1) * RT / 10) issue_j(si, 4 + i);
+          }
           __builtin_amdgcn_sched_barrier(0);
           b_last = bcur;
         }
@@ -2319,11 +2487,13 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
 
       bool abort = false;
       if (nst > 0) {  // ---- iteration 0: QK and softmax of stage 0, all loads of stage 2
-        if (1 < nst) wait_vmcnt<9>();  // stage 0 landed; stage 1 may stay in flight
+        if constexpr (KV8) wait_vmcnt<5>();  // stage 1 landed; stage 2's codes may stay in flight
+        else if (1 < nst) wait_vmcnt<9>();   // stage 0 landed; stage 1 may stay in flight
         else wait_vmcnt<0>();
         wait_lgkm0();
         lds_barrier();
-        if (2 < nst) issue(2);
+        if constexpr (!KV8)
+          if (2 < nst) issue(2);
         const int ln0 = fresh_lane();
         const LaneOffsets lo = lane_offsets(ln0);
         f32x4 acc[HT][2];
@@ -2337,9 +2507,15 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         } else {
           if constexpr (MODE == kPassFirstStageRef) {
 #pragma unroll
-            for (int ht = 0; ht < HT; ++ht) m_ref[ht] = wave_max_g(lmx[ht]);
+            for (int ht = 0; ht < HT; ++ht) m_ref[ht] = fmaxf(wave_max_g(lmx[ht]), kMinRef);
           }
           softmax_publish(0, acc);
+        }
+        if constexpr (KV8) {  // stage 2's rope, stage 1 dequantised, stage 3's codes
+          si = prepare(3, si);
+          issue_one(si, std::integral_constant<int, 0>{});
+          dequant(1);
+          issue_codes(si);
         }
       }
       // ---- k = 1 .. nst
@@ -2348,12 +2524,13 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       const int kend = kPV ? nst + 1 : nst;
       // the loads of stage k + 2, prepared at the end of iteration k - 1 (while the wave waits
       // for its P^T stores before the barrier) rather than between the barrier and QK
-      StageIssue si;
-      if constexpr (kPrepEarly) si = prepare(3);
+      if constexpr (kPrepEarly) si = prepare(1 + kLead, si);
 #pragma unroll 1
       for (int k = 1; k < kend; ++k) {
         const bool has_qk = k < nst;  // uniform
-        if (has_qk) {
+        if constexpr (KV8) {
+          wait_vmcnt<6>();  // stage k + 1's codes and stage k's rope landed (dummies past the segment)
+        } else if (has_qk) {
           if (k + 1 < nst) wait_vmcnt<9>();  // stage k landed; stage k+1 may stay in flight
           else wait_vmcnt<0>();
         }
@@ -2368,7 +2545,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         }
         uint32_t vm = ~0u;
         if constexpr (SPARSE) vm = (uint32_t)__builtin_amdgcn_readfirstlane((int)vmask_sh[k]);
-        if constexpr (!kPrepEarly) si = prepare(k + 2);  // past the segment: dummy loads
+        if constexpr (!kPrepEarly) si = prepare(k + kLead, si);  // past the segment: dummy loads
         // 64-row form: from a fresh lane id per iteration (kept live across the loop they
         // spill); 128-row form: once per pass (no spill there, 27 fewer VALU per stage)
         const LaneOffsets lo = HT == 1 ? lane_offsets(fresh_lane()) : lo_pass;
@@ -2418,6 +2595,9 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         }
         if constexpr (kPV) {
           pv_softmax(k - 1, acc, va, bq, si, lo, vm, over);
+        } else if constexpr (KV8) {
+          dequant(k + 1);
+          issue_codes(si);
         } else {
 #pragma unroll
           for (int j = 4; j < 9; ++j) issue_j(si, j);
@@ -2425,7 +2605,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         if constexpr (MODE == kPassFirstStageRef) {
           if (__builtin_amdgcn_ballot_w64(over) != 0) over_sh[k & 3] = 1;  // uniform branch
         }
-        if constexpr (kPrepEarly) si = prepare(k + 3);  // past the segment: dummy loads (see prepare)
+        if constexpr (kPrepEarly) si = prepare(k + 1 + kLead, si);  // past the segment: dummy loads (see prepare)
       }
       wait_vmcnt<0>();  // an abandoned pass may leave stage loads in flight
       wait_lgkm0();
@@ -3603,7 +3783,9 @@ hipError_t launch_main(const mla::KParams& kp, int head_blocks, hipStream_t st) 
 }
 
 // The 64- and 128-row decodes over a 16-bit cache run the wide kernel (PV split by dims across the
-// waves) unless MLA_WIDE=0 selects the one-ring four-wave kernel (which the fp8 cache runs).
+// waves) unless MLA_WIDE=0 selects the one-ring four-wave kernel, and so do those over the paged fp8
+// cache; the sparse decode over it keeps the one-ring kernel (its three row addresses per lane do
+// not fit the 128-row form).
 bool wide_enabled() {
   static std::once_flag once;
   static bool on = true;
@@ -3614,14 +3796,14 @@ bool wide_enabled() {
   return on;
 }
 
-template <int DT, int HT, bool FUSED, bool SPARSE>
+template <int DT, int HT, bool FUSED, bool SPARSE, bool KV8 = false>
 void launch_wide_form(const mla::KParams& kp, int head_blocks, hipStream_t st) {
   const int wgs = kp.num_parts * head_blocks;
   if (wgs % 8 == 0) {  // XCD-blocked 1-D grid (see the kernel)
-    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED, SPARSE>), dim3(wgs), dim3(256), 0, st, kp.sched, head_blocks,
+    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED, SPARSE, KV8>), dim3(wgs), dim3(256), 0, st, kp.sched, head_blocks,
                        wgs / 8, kp);
   } else {
-    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED, SPARSE>), dim3(kp.num_parts, head_blocks), dim3(256), 0, st,
+    hipLaunchKernelGGL((mla::mla_wide_kernel<DT, HT, FUSED, SPARSE, KV8>), dim3(kp.num_parts, head_blocks), dim3(256), 0, st,
                        kp.sched, 0, 0, kp);
   }
 }
@@ -3661,6 +3843,11 @@ hipError_t launch_main_dt(const Variant& v, const mla::KParams& kp, int head_blo
     if (kp.kv_scale != nullptr) {  // fp8 latent cache
       if (v.ws) return launch_main<DT, 4, 1, 1, true, true>(kp, head_blocks, st);
       if (v.nw == 1) return launch_main<DT, 1, 2, 1, false, true>(kp, head_blocks, st);
+      if (wide_enabled() && kp.ks_sb < (1 << 28)) {  // a lane's scale offset is formed in 32 bits
+        if (v.ht == 1) launch_wide_form<DT, 1, false, false, true>(kp, head_blocks, st);
+        else launch_wide_form<DT, 2, false, false, true>(kp, head_blocks, st);
+        return hipGetLastError();
+      }
       if (v.ht == 1) return launch_main<DT, 4, 1, 4, false, true>(kp, head_blocks, st);
       return launch_main<DT, 4, 2, 3, false, true>(kp, head_blocks, st);
     }

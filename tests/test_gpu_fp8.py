@@ -203,3 +203,34 @@ def test_fp8_append_then_decode(gpu):
     deq = F8.dequantize_pages(lat2, sc2, rope2)
     ref_out, ref_lse = R.decode_paged(inp.q, deq, inp.block_table, lens2, inp.sm_scale, True)
     assert_parity(out, lse, ref_out, ref_lse, "fp8 append then decode")
+
+
+@pytest.mark.parametrize("H,s_q", [(40, 1), (64, 1), (128, 1), (100, 2)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_fp8_wide_stages(gpu, H, s_q, padded):
+    """More than 32 query rows: one to many stages per segment (the raw and bf16 rings wrap, and a
+    segment passes a 64-page window), segments redone for a score far above their first stage's
+    (the rope dims of every token past the 32nd scaled up; V kept below 2, where half a bf16 ulp
+    is 0.004), and caches that are views of wider tensors."""
+    lens = [1, 32, 33, 64, 97, 5000]
+    cfg = small_cfg(f"fp8_wide_{H}", len(lens), s_q, H, lens)
+    inp = make_inputs(cfg, seed=H + s_q)
+    inp.kv_cache[..., :512] *= 0.25
+    for redo in (False, True):
+        if redo:
+            for b, n in enumerate(lens):
+                t = torch.arange(min(32, n), n)
+                inp.kv_cache[inp.block_table[b, t // 64].long(), t % 64, 0, 512:] *= 100
+        lat, sc, rope = F8.quantize_pages(inp.kv_cache)
+        deq = F8.dequantize_pages(lat, sc, rope)
+        cache = to_gpu_fp8(lat, sc, rope)
+        if padded:
+            nb = rope.shape[0]
+            wide = [torch.zeros(nb, 64, 528, dtype=torch.uint8, device="cuda"), torch.zeros(nb, 5, 68, device="cuda"),
+                    torch.zeros(nb, 66, 72, dtype=torch.bfloat16, device="cuda")]
+            views = (wide[0][:, :, :512], wide[1][:, :4, :64], wide[2][:, :64, :64])
+            for v, t in zip(views, cache):
+                v.copy_(t)
+            cache = Fp8KVCache(*views)
+        for ns in (None, 1):
+            check_fp8(inp, cache, deq, num_splits=ns, what=f"fp8 wide H={H} s_q={s_q} padded={padded} redo={redo} ns={ns}")
