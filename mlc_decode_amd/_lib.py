@@ -152,6 +152,8 @@ def library_path() -> str:
 def load() -> ctypes.CDLL:
     """Load the built library (once).  Raises if it has not been built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

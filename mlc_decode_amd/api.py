@@ -22,8 +22,10 @@ int32, cache_seqlens ``[B]`` int32, out ``[B, s_q, H, 512]`` in q's dtype and ls
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import math
+import struct
 import threading
 from typing import NamedTuple, Optional, Sequence, Tuple, Union
 
@@ -36,11 +38,25 @@ from ._lib import (MLA_DIM_QK, MLA_DIM_V, MLA_DTYPE_BF16, MLA_DTYPE_F16, MLA_KV_
 _DTYPES = {torch.bfloat16: MLA_DTYPE_BF16, torch.float16: MLA_DTYPE_F16}
 
 _ws_lock = threading.Lock()
-_workspaces: dict = {}   # (device index, stream handle) -> the buffer calls on that stream use
+_workspaces: dict = {}   # (device index, stream handle) -> (buffer, aligned address, bytes) of calls on that stream
 _retired: list = []      # buffers replaced by larger ones, kept alive until the process ends
 
 
+# The argument structs are filled by one struct.pack each: setting some forty ctypes fields one by
+# one took longer than launching the kernels.
+_DECODE_ARGS = struct.Struct("=6ifiQQ6qQQ6qQ2i3QQ3qQQq2iQ2qQ2i2iQ")
+_APPEND_ARGS = struct.Struct("=4iQ2qQQ4qQ2iQQ2iQ2q")
+assert _DECODE_ARGS.size == ctypes.sizeof(MlaDecodeArgs) and _APPEND_ARGS.size == ctypes.sizeof(MlaKvAppendArgs)
+
+_FLT_MAX = 3.4028234663852886e38
+
+# torch's raw handle of the current stream, without the Stream object around it where torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -61,21 +77,33 @@ def workspace(device: torch.device, nbytes: int, stream: Optional[torch.cuda.Str
     the retired buffers of a stream together hold less than its live one.  The returned
     slice's length is the byte count to pass as ``workspace_bytes``.
     """
-    nbytes = max(int(nbytes), 256)
     if stream is None:
         stream = torch.cuda.current_stream(device)
     index = device.index if device.index is not None else torch.cuda.current_device()
-    key = (index, stream.cuda_stream)
+    buf, ptr, _ = _workspace(torch.device(device.type, index), stream.cuda_stream, int(nbytes))
+    return buf[ptr - buf.data_ptr():]
+
+
+def _workspace(device: torch.device, stream: int, nbytes: int):
+    """``workspace`` by stream handle: ``(buffer, aligned address, bytes from there)``."""
+    nbytes = max(nbytes, 256)
+    key = (device.index, stream)
     with _ws_lock:
-        buf = _workspaces.get(key)
-        if buf is None or buf.numel() - (-buf.data_ptr()) % 256 < nbytes:
-            size = grown_workspace_size(None if buf is None else buf.numel(), nbytes + 256)
-            if buf is not None:
-                _retired.append(buf)
+        ws = _workspaces.get(key)
+        if ws is None or ws[2] < nbytes:
+            size = grown_workspace_size(None if ws is None else ws[0].numel(), nbytes + 256)
+            if ws is not None:
+                _retired.append(ws[0])
             buf = torch.empty(size, dtype=torch.uint8, device=device)
-            _workspaces[key] = buf
-    off = (-buf.data_ptr()) % 256
-    return buf[off:]
+            off = (-buf.data_ptr()) % 256
+            ws = (buf, buf.data_ptr() + off, size - off)
+            _workspaces[key] = ws
+    return ws
+
+
+@functools.lru_cache(maxsize=4096)
+def _workspace_bytes(batch: int, s_q: int, heads: int, num_parts: int) -> int:
+    return _lib.load().mla_workspace_bytes(batch, s_q, heads, num_parts)
 
 
 def grown_workspace_size(current: Optional[int], need: int) -> int:
@@ -89,6 +117,7 @@ def grown_workspace_size(current: Optional[int], need: int) -> int:
     return size
 
 
+@functools.lru_cache(maxsize=4096)
 def num_parts_for(batch: int, s_q: int, heads_q: int, heads_k: int = 1, cu_count: int = 0) -> int:
     """Schedule parts the decode kernel is laid out for (``mla_num_parts``)."""
     n = _lib.load().mla_num_parts(batch, s_q, heads_q, heads_k, cu_count)
@@ -194,6 +223,15 @@ def quantize_kv_cache(kv_cache: torch.Tensor) -> Fp8KVCache:
     return dst
 
 
+def _check_native_cache(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
+    _require_gpu(t, name)
+    if t.dtype != dtype:
+        raise ValueError("kv cache dtype must match q")
+    shape = t.shape
+    if len(shape) != 4 or shape[1] != _lib.MLA_PAGE_TOKENS or shape[2] != 1 or t.stride(-1) != 1:
+        raise ValueError("kv cache must be [num_blocks, 64, 1, D] with unit stride in D")
+
+
 def _split_kv(kv_cache) -> Tuple[torch.Tensor, torch.Tensor]:
     if isinstance(kv_cache, Fp8KVCache):
         raise ValueError("an fp8 cache has no bf16 latent half")
@@ -223,22 +261,33 @@ def make_decode_args(q: torch.Tensor, kv_cache, block_table: Optional[torch.Tens
     _require_gpu(q, "q")
     if q.dim() != 4 or q.shape[-1] != MLA_DIM_QK:
         raise ValueError(f"q must be [B, s_q, H, {MLA_DIM_QK}]")
-    if q.dtype not in _DTYPES:
+    dtype = q.dtype
+    if dtype not in _DTYPES:
         raise ValueError("q must be bfloat16 or float16")
     fp8 = isinstance(kv_cache, Fp8KVCache)
+    scale, scale_ptr, scale_page, scale_blk = None, 0, 0, 0
     if fp8:
         latent, scale, rope = _check_fp8_cache(kv_cache)
-        if q.dtype != torch.bfloat16:
+        if dtype != torch.bfloat16:
             raise ValueError("the fp8 cache is read with bf16 queries")
-    else:
+        (kv_page, kv_tok, _), (kr_page, kr_tok, _) = latent.stride(), rope.stride()
+        kv_ptr, kr_ptr = latent.data_ptr(), rope.data_ptr()
+        scale_ptr = scale.data_ptr()
+        scale_page, scale_blk, _ = scale.stride()
+    elif isinstance(kv_cache, (tuple, list)):
         latent, rope = _split_kv(kv_cache)
-        scale = None
         for t, n in ((latent, "kv latent"), (rope, "kv rope")):
-            _require_gpu(t, n)
-            if t.dtype != q.dtype:
-                raise ValueError("kv cache dtype must match q")
-            if t.dim() != 4 or t.shape[1] != _lib.MLA_PAGE_TOKENS or t.shape[2] != 1 or t.stride(-1) != 1:
-                raise ValueError("kv cache must be [num_blocks, 64, 1, D] with unit stride in D")
+            _check_native_cache(t, n, dtype)
+        kv_page, kv_tok, kr_page, kr_tok = latent.stride(0), latent.stride(1), rope.stride(0), rope.stride(1)
+        kv_ptr, kr_ptr = latent.data_ptr(), rope.data_ptr()
+    else:  # one tensor: the rope half starts 512 elements into each row
+        latent = rope = kv_cache
+        if kv_cache.shape[-1] != MLA_DIM_QK:
+            raise ValueError(f"kv_cache last dim must be {MLA_DIM_QK}")
+        _check_native_cache(kv_cache, "kv latent", dtype)
+        kv_page, kv_tok = kr_page, kr_tok = kv_cache.stride()[:2]
+        kv_ptr = kv_cache.data_ptr()
+        kr_ptr = kv_ptr + MLA_DIM_V * 2
     B, s_q, H, _ = q.shape
     if indices is not None:  # sparse: keys named by index, no page table or lengths
         _require_gpu(indices, "indices")
@@ -261,7 +310,8 @@ def make_decode_args(q: torch.Tensor, kv_cache, block_table: Optional[torch.Tens
             raise ValueError("cache_seqlens must be a 1-D int32 tensor")
         if block_table.shape[0] != B or cache_seqlens.shape[0] != B or splits.numel() != B + 1:
             raise ValueError("batch size of q, block_table, cache_seqlens and num_splits disagree")
-    if q.stride(-1) != 1:
+    qs_b, qs_s, qs_h, qs_d = q.stride()
+    if qs_d != 1:
         raise ValueError("q must have unit stride in its last dim")
     if status is not None:
         _require_gpu(status, "status")
@@ -279,46 +329,29 @@ def make_decode_args(q: torch.Tensor, kv_cache, block_table: Optional[torch.Tens
     sched = sched.contiguous()
     splits = splits.contiguous()
     num_parts = sched.shape[0]
-    lib = _lib.load()
-    ws = workspace(q.device, lib.mla_workspace_bytes(B, s_q, H, num_parts))
-    el = q.element_size()
-    a = MlaDecodeArgs()
-    a.batch, a.s_q, a.heads_q, a.heads_k = B, s_q, H, 1
-    a.dtype = _DTYPES[q.dtype]
-    a.causal = 1 if causal else 0
-    a.sm_scale = float(sm_scale)
-    a.num_blocks = latent.shape[0]
-    a.q_nope = q.data_ptr()
-    a.q_rope = q.data_ptr() + MLA_DIM_V * el
-    a.q_stride_b, a.q_stride_s, a.q_stride_h = q.stride(0), q.stride(1), q.stride(2)
-    a.q_rope_stride_b, a.q_rope_stride_s, a.q_rope_stride_h = q.stride(0), q.stride(1), q.stride(2)
-    a.kv_nope, a.kv_rope = latent.data_ptr(), rope.data_ptr()
-    a.kv_stride_page, a.kv_stride_tok, a.kv_stride_batch = latent.stride(0), latent.stride(1), 0
-    a.kv_rope_stride_page, a.kv_rope_stride_tok, a.kv_rope_stride_batch = rope.stride(0), rope.stride(1), 0
-    a.kv_format = MLA_KV_FP8_E4M3 if fp8 else MLA_KV_NATIVE
-    if fp8:
-        a.kv_scale = scale.data_ptr()
-        a.kv_scale_stride_page, a.kv_scale_stride_blk = scale.stride(0), scale.stride(1)
+    device = q.device
+    ws, ws_ptr, ws_bytes = _workspace(device, _stream_ptr(device), _workspace_bytes(B, s_q, H, num_parts))
+    q_ptr = q.data_ptr()
     if indices is not None:
-        a.indices = indices.data_ptr()
-        a.indices_stride, a.topk = indices.stride(0), indices.shape[1]
-        a.block_table, a.block_table_stride = None, 0
-        a.kv_stride_batch = a.kv_rope_stride_batch = 0
+        idx_ptr, idx_stride, topk = indices.data_ptr(), indices.stride(0), indices.shape[1]
+        bt_ptr = bt_stride = bt_width = 0
     else:
-        a.block_table = block_table.data_ptr()
+        idx_ptr = idx_stride = topk = 0
+        bt_ptr, bt_width = block_table.data_ptr(), block_table.shape[1]
         # one row: its stride is never used, and a view's may be anything
-        a.block_table_stride = block_table.stride(0) if B > 1 else block_table.shape[1]
-        a.block_table_width = block_table.shape[1]
-    a.status = status.data_ptr() if status is not None else None
-    a.num_parts = num_parts
-    a.cache_seqlens = seqlens.data_ptr() if seqlens is not None else None
-    a.tile_sched = sched.data_ptr()
-    a.num_splits = splits.data_ptr()
-    a.out = out.data_ptr()
-    a.o_stride_b, a.o_stride_s, a.o_stride_h = out.stride(0), out.stride(1), out.stride(2)
-    a.lse = lse.data_ptr()
-    a.workspace = ws.data_ptr()
-    a.workspace_bytes = ws.numel()
+        bt_stride = block_table.stride(0) if B > 1 else bt_width
+    os_b, os_s, os_h, _ = out.stride()
+    sm_scale = float(sm_scale)
+    if abs(sm_scale) > _FLT_MAX:  # as a C float: refused there
+        sm_scale = math.copysign(math.inf, sm_scale)
+    a = MlaDecodeArgs.from_buffer_copy(_DECODE_ARGS.pack(
+        B, s_q, H, 1, _DTYPES[dtype], 1 if causal else 0, sm_scale, latent.shape[0],
+        q_ptr, q_ptr + MLA_DIM_V * 2, qs_b, qs_s, qs_h, qs_b, qs_s, qs_h,
+        kv_ptr, kr_ptr, kv_page, kv_tok, 0, kr_page, kr_tok, 0,
+        bt_ptr, bt_stride, num_parts, seqlens.data_ptr() if seqlens is not None else 0, sched.data_ptr(),
+        splits.data_ptr(), out.data_ptr(), os_b, os_s, os_h, lse.data_ptr(), ws_ptr, ws_bytes,
+        MLA_KV_FP8_E4M3 if fp8 else MLA_KV_NATIVE, 0, scale_ptr, scale_page, scale_blk,
+        idx_ptr, idx_stride, topk, bt_width, 0, status.data_ptr() if status is not None else 0))
     keep = (q, latent, rope, scale, block_table, seqlens, sched, splits, out, lse, ws, indices, status)
     return a, out, lse, keep
 
@@ -478,10 +511,16 @@ def kv_append(kv_new: torch.Tensor, kv_cache, block_table: torch.Tensor,
     """
     _require_gpu(kv_new, "kv_new")
     fp8 = isinstance(kv_cache, Fp8KVCache)
+    rope_offset = 0
     if fp8:
         latent, scale, rope = _check_fp8_cache(kv_cache)
-    else:
+    elif isinstance(kv_cache, (tuple, list)):
         latent, rope = _split_kv(kv_cache)
+    else:  # one tensor: the rope half starts 512 elements into each row
+        if kv_cache.shape[-1] != MLA_DIM_QK:
+            raise ValueError(f"kv_cache last dim must be {MLA_DIM_QK}")
+        latent = rope = kv_cache
+        rope_offset = MLA_DIM_V * 2
     if kv_new.dim() == 4:
         if kv_new.shape[2] != 1:
             raise ValueError("kv_new [B, n_new, 1, 576] must have one KV head")
@@ -506,21 +545,13 @@ def kv_append(kv_new: torch.Tensor, kv_cache, block_table: torch.Tensor,
         raise ValueError("status must be an int32 tensor of at least one element")
     for t, name in ((latent, "kv_cache"), (block_table, "block_table"), (cache_seqlens, "cache_seqlens")):
         _require_gpu(t, name)
-    a = MlaKvAppendArgs()
-    a.batch, a.n_new, a.dtype, a.num_blocks = B, n_new, _DTYPES[kv_new.dtype], latent.shape[0]
-    a.kv_new = kv_new.data_ptr()
-    a.new_stride_b, a.new_stride_t = kv_new.stride(0), kv_new.stride(1)
-    a.kv_nope, a.kv_rope = latent.data_ptr(), rope.data_ptr()
-    a.kv_stride_page, a.kv_stride_tok = latent.stride(0), latent.stride(1)
-    a.kv_rope_stride_page, a.kv_rope_stride_tok = rope.stride(0), rope.stride(1)
-    a.block_table = block_table.data_ptr()
-    a.block_table_stride, a.max_pages = block_table.stride(0), block_table.shape[1]
-    a.cache_seqlens = cache_seqlens.data_ptr()
-    a.status = status.data_ptr() if status is not None else None
-    if fp8:
-        a.kv_format = MLA_KV_FP8_E4M3
-        a.kv_scale = scale.data_ptr()
-        a.kv_scale_stride_page, a.kv_scale_stride_blk = scale.stride(0), scale.stride(1)
+    (new_b, new_t, _), (kv_page, kv_tok), (kr_page, kr_tok) = kv_new.stride(), latent.stride()[:2], rope.stride()[:2]
+    scale_args = (MLA_KV_FP8_E4M3, 0, scale.data_ptr(), *scale.stride()[:2]) if fp8 else (MLA_KV_NATIVE, 0, 0, 0, 0)
+    a = MlaKvAppendArgs.from_buffer_copy(_APPEND_ARGS.pack(
+        B, n_new, _DTYPES[kv_new.dtype], latent.shape[0], kv_new.data_ptr(), new_b, new_t,
+        latent.data_ptr(), rope.data_ptr() + rope_offset, kv_page, kv_tok, kr_page, kr_tok,
+        block_table.data_ptr(), block_table.stride(0) if B > 1 else min(block_table.stride(0), 2 ** 31 - 1), block_table.shape[1], cache_seqlens.data_ptr(),
+        status.data_ptr() if status is not None else 0, *scale_args))
     check("mla_kv_append", _lib.load().mla_kv_append(ctypes.byref(a), _stream_ptr(kv_new.device)))
     return a
 
