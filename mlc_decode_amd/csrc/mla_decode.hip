@@ -2830,12 +2830,12 @@ __global__ __launch_bounds__(SW == 16 ? 1024 : 256) void mla_kv_append_kernel(Ap
     }
   }
   const int L = a.seqlens[b];
-  const int pos_l = (int)((uint32_t)L + (uint32_t)lane);  // token `lane`'s position
+  const int pos_l = SW == 1 ? L : (int)((uint32_t)L + (uint32_t)lane);  // token `lane`'s position
   int page = -1;
-  if (lane < a.n_new && L >= 0 && pos_l >= 0 && (pos_l >> 6) < a.max_pages)
+  if ((SW == 1 || lane < a.n_new) && L >= 0 && pos_l >= 0 && (pos_l >> 6) < a.max_pages)
     page = a.block_table[(int64_t)b * a.bt_stride + (pos_l >> 6)];
-  const bool bad = lane < a.n_new && (page < 0 || page >= a.num_blocks);
-  const bool ok = __builtin_amdgcn_ballot_w64(bad) == 0;  // uniform, the same in every wave
+  const bool bad = (SW == 1 || lane < a.n_new) && (page < 0 || page >= a.num_blocks);
+  const bool ok = SW == 1 ? !bad : __builtin_amdgcn_ballot_w64(bad) == 0;  // uniform, the same in every wave
   if constexpr (SW > 1) __syncthreads();  // every wave has read the length
   if (w == 0 && lane == 0) {
     if (ok)
@@ -2848,7 +2848,7 @@ __global__ __launch_bounds__(SW == 16 ? 1024 : 256) void mla_kv_append_kernel(Ap
   for (int i = 0; i < kTok; ++i) {
     const int t = w + SW * i;
     if (t >= a.n_new) break;  // uniform
-    const int pg = __builtin_amdgcn_readlane(page, t);
+    const int pg = SW == 1 ? page : __builtin_amdgcn_readlane(page, t);
     const int row = (L + t) & 63;
     if (a.kv8) {  // uniform
       // lane l holds dims 8l .. 8l+7; block j (dims 128j ..) is the lane group of 16
@@ -3072,10 +3072,14 @@ constexpr int kDeepSplits = 256;
 constexpr int kDeepMaxRows = 16384;  // kDeepSplits * kDeepMaxRows KiB = 2^32 bytes
 constexpr int kQueue = 32;
 constexpr int kDeepLds = (kDeepSplits + kQueue) * 4;  // kw
+constexpr int kShareSplits = 64;  // longer rows are shared by a workgroup's waves (see launch_combine)
+// Splits lo .. hi - 1 only, with the weights of a merge of all n: the waves of a workgroup that
+// share a quarter row take consecutive ranges of its splits, and their sums are added.
 template <int DT, bool SCALED>
 __device__ __forceinline__ float merge_many_splits(const uint16_t* __restrict__ ws_o, const float* __restrict__ ws_scale,
                                                    const float* __restrict__ ws_lse, int base, int n, int rows,
-                                                   int row, int q, int lane, char* smem, float (&acc)[2]) {
+                                                   int row, int q, int lane, char* smem, int lo, int hi,
+                                                   float (&acc)[2]) {
   static_assert(kDeepSplits % 64 == 0 && kQueue <= 63 && kQueue % 4 == 0 && kQueue <= 64, "queue shape");
   constexpr int LDT = SCALED ? MLA_DTYPE_F16 : DT;
   constexpr int kL = kDeepSplits / 64;
@@ -3087,9 +3091,9 @@ __device__ __forceinline__ float merge_many_splits(const uint16_t* __restrict__ 
   const char* row0 = (const char*)(ws_o + ((int64_t)base * rows + row) * kDV + 128 * q);
   const uint32_t split_bytes = (uint32_t)rows * kDV * 2;
   const float* lp = ws_lse + (int64_t)base * rows + row;
-  const int last = n - 1;
+  const int last = (lo < hi ? hi : n) - 1;  // the last split this wave loads
   const uint32_t last_off = (uint32_t)last * split_bytes;
-  uint32_t next_off = 0;  // the next split to load, clamped to the last
+  uint32_t next_off = (uint32_t)(lo < last ? lo : last) * split_bytes;  // the next split to load, clamped to the last
   auto load_next = [&]() __attribute__((always_inline)) {
     const uint32_t v = *(const uint32_t*)(row0 + next_off + lane * 4);
     next_off = next_off + split_bytes < last_off ? next_off + split_bytes : last_off;
@@ -3100,7 +3104,7 @@ __device__ __forceinline__ float merge_many_splits(const uint16_t* __restrict__ 
 #pragma unroll
   for (int c = 0; c < kL; ++c) {
     const int k = c * 64 + lane;
-    const int kc = k < last ? k : last;
+    const int kc = k < n - 1 ? k : n - 1;
     const float l = lp[(int64_t)kc * rows];
     lv[c] = k < n ? l : -INFINITY;
     if constexpr (SCALED) sc[c] = ws_scale[((int64_t)(base + kc) * rows + row) * 4 + q];
@@ -3142,7 +3146,7 @@ __device__ __forceinline__ float merge_many_splits(const uint16_t* __restrict__ 
       for (int u = u4; u < u4 + 4; ++u) {
         // in the last block a row past the last split is zeroed: acc + 0 * 0 = acc exactly
         // (acc is never -0)
-        const uint32_t v = (decltype(tail)::value && k0 + u >= n) ? 0u : qv[u];
+        const uint32_t v = (decltype(tail)::value && k0 + u >= hi) ? 0u : qv[u];
         float x0, x1;
         if constexpr (LDT == MLA_DTYPE_BF16) {
           x0 = __builtin_bit_cast(float, v << 16);
@@ -3158,8 +3162,8 @@ __device__ __forceinline__ float merge_many_splits(const uint16_t* __restrict__ 
       }
     }
   };
-  for (int k0 = 0; k0 < n; k0 += kQueue) {
-    if (k0 + kQueue <= n)  // uniform
+  for (int k0 = lo; k0 < hi; k0 += kQueue) {
+    if (k0 + kQueue <= hi)  // uniform
       block(k0, std::false_type{});
     else
       block(k0, std::true_type{});
@@ -3167,13 +3171,13 @@ __device__ __forceinline__ float merge_many_splits(const uint16_t* __restrict__ 
   return lse2;
 }
 
-// One wave per (sequence, row).  DEEP (chosen by the host when the batch is small next to the
-// part count, so sequences have many splits and the grid is small): one wave per workgroup and
-// grid.z = 4, the quarter of the row the wave merges when the row has kFewSplits < n <=
-// kDeepSplits splits (merge_many_splits); other rows are merged whole by quarter 0.  Otherwise
-// four waves per workgroup, for large batches of rows with few splits each.
-template <int DT, typename PT, bool SCALED, bool DEEP = false>
-__global__ __launch_bounds__(DEEP ? 64 : 256) void mla_combine_kernel(const PT* __restrict__ ws_o,
+// One wave per (sequence, row).  DEEP > 0 (chosen by the host when the batch is small next to the
+// part count, so sequences have many splits and the grid is small): DEEP waves per workgroup and
+// grid.z = 4, the quarter of the row the workgroup merges when the row has kFewSplits < n <=
+// kDeepSplits splits (merge_many_splits); other rows are merged whole by the first wave of quarter
+// 0.  Otherwise four waves per workgroup, for large batches of rows with few splits each.
+template <int DT, typename PT, bool SCALED, int DEEP = 0>
+__global__ __launch_bounds__(DEEP ? 64 * DEEP : 256) void mla_combine_kernel(const PT* __restrict__ ws_o,
                                                           const float* __restrict__ ws_scale,
                                                           const float* __restrict__ ws_lse,
                                                           const int32_t* __restrict__ splits,
@@ -3182,13 +3186,14 @@ __global__ __launch_bounds__(DEEP ? 64 : 256) void mla_combine_kernel(const PT* 
                                                           int64_t o_sb, int64_t o_ss, int64_t o_sh,
                                                           float* __restrict__ lse_out,
                                                           int copy_single) {
-  constexpr int W = DEEP ? 1 : 4;  // waves (rows) per workgroup
-  __shared__ __attribute__((aligned(16))) char smem[DEEP ? kDeepLds : W * 64 * 4];
-  float* w_sh = (float*)smem + 64 * (threadIdx.x >> 6);  // the wave's 64 weights (merge_splits_wave)
+  constexpr int W = DEEP ? 1 : 4;  // rows per workgroup
+  __shared__ __attribute__((aligned(16))) char smem[DEEP ? DEEP * kDeepLds : W * 64 * 4];
+  __shared__ float sum_sh[DEEP > 1 ? DEEP : 1][2][64];
+  float* w_sh = (float*)smem + (DEEP ? 0 : 64 * (threadIdx.x >> 6));  // the wave's 64 weights (merge_splits_wave)
   const int b = blockIdx.x;
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.y * W + wave;
+  const int row = blockIdx.y * W + (DEEP ? 0 : wave);
   if (row >= rows) return;
   const int base = splits[b];
   const int n = splits[b + 1] - base;
@@ -3197,16 +3202,33 @@ __global__ __launch_bounds__(DEEP ? 64 : 256) void mla_combine_kernel(const PT* 
   const int h = row - s * heads;
   uint16_t* dst = out + b * o_sb + s * o_ss + h * o_sh;
   float* lse_dst = lse_out != nullptr ? lse_out + ((int64_t)b * heads + h) * s_q + s : nullptr;
-  if constexpr (DEEP && std::is_same<PT, uint16_t>::value) {
+  if constexpr (DEEP > 0 && std::is_same<PT, uint16_t>::value) {
     const int q = blockIdx.z;
     if (n > kFewSplits && n <= kDeepSplits) {  // uniform
       float acc2[2];
-      const float lse2 = merge_many_splits<DT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, q, lane, smem, acc2);
+      const bool share = DEEP > 1 && n > kShareSplits;  // uniform
+      if (!share && wave != 0) return;
+      const int per = share ? ((n + 4 * DEEP - 1) / (4 * DEEP)) * 4 : n;  // whole fours: the weights are read so
+      const int lo = wave * per;
+      const int hi = lo + per < n ? lo + per : n;
+      const float lse2 = merge_many_splits<DT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, q, lane,
+                                                       smem + wave * kDeepLds, lo, hi, acc2);
+      if (share) {
+        sum_sh[wave][0][lane] = acc2[0];
+        sum_sh[wave][1][lane] = acc2[1];
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int v = 1; v < DEEP; ++v) {
+          acc2[0] += sum_sh[v][0][lane];
+          acc2[1] += sum_sh[v][1][lane];
+        }
+      }
       *(uint32_t*)(dst + 128 * q + 2 * lane) = pack2<DT>(acc2[0], acc2[1]);
       if (q == 0 && lane == 0 && lse_dst != nullptr) *lse_dst = lse2 * kLn2;
       return;
     }
-    if (q != 0) return;
+    if (q != 0 || wave != 0) return;
   }
   float acc[8];
   float lse2;
@@ -3989,17 +4011,30 @@ bool combine_is_deep(const mla::KParams& k) {
 
 template <typename PT, bool SCALED = false>
 int launch_combine(const mla::KParams& k, const PT* part_o, int dtype, int copy_single, hipStream_t st) {
-  const bool deep = std::is_same<PT, uint16_t>::value && combine_is_deep(k);
+  // Four waves share a quarter row's splits where its merge is long (more than 64) and the rows are
+  // so few that one wave each leaves most of the chip idle.  Combine alone, one -> four waves: 16
+  // rows x 256 splits 7.1 -> 4.9 us, 128 x 256 10.1 -> 9.1, 32 x 128 5.3 -> 4.3; but 128 x 64 splits
+  // 4.3 -> 5.0, 128 x 32 3.9 -> 4.9, 256 rows x 128 7.0 -> 8.9.
+  const bool share = (int64_t)k.batch * k.rows <= 128 && k.num_parts > mla::kShareSplits * (int64_t)k.batch;
+  const int deep = !(std::is_same<PT, uint16_t>::value && combine_is_deep(k)) ? 0 : share ? 4 : 1;
   const int W = deep ? 1 : 4;
   const dim3 grid(k.batch, (k.rows + W - 1) / W, deep ? 4 : 1);
-#define MLA_COMBINE(D, DP)                                                                                      \
-  hipLaunchKernelGGL((mla::mla_combine_kernel<D, PT, SCALED, DP>), grid, dim3(64 * W), 0, st, part_o, k.ws_scale, \
-                     k.ws_lse, k.splits, k.rows, k.heads, k.s_q, k.out, k.o_sb, k.o_ss, k.o_sh, k.lse, copy_single)
-  if (dtype == MLA_DTYPE_BF16) {
-    if (deep) MLA_COMBINE(MLA_DTYPE_BF16, true); else MLA_COMBINE(MLA_DTYPE_BF16, false);
-  } else {
-    if (deep) MLA_COMBINE(MLA_DTYPE_F16, true); else MLA_COMBINE(MLA_DTYPE_F16, false);
-  }
+#define MLA_COMBINE(D, DP)                                                                                     \
+  hipLaunchKernelGGL((mla::mla_combine_kernel<D, PT, SCALED, DP>), grid, dim3(DP ? 64 * DP : 256), 0, st, part_o, \
+                     k.ws_scale, k.ws_lse, k.splits, k.rows, k.heads, k.s_q, k.out, k.o_sb, k.o_ss, k.o_sh, k.lse, \
+                     copy_single)
+#define MLA_COMBINE_DT(D)                      \
+  do {                                         \
+    if constexpr (!std::is_same<PT, uint16_t>::value) { MLA_COMBINE(D, 0); } \
+    else if (deep == 4) MLA_COMBINE(D, 4);     \
+    else if (deep == 1) MLA_COMBINE(D, 1);     \
+    else MLA_COMBINE(D, 0);                    \
+  } while (0)
+  if (dtype == MLA_DTYPE_BF16)
+    MLA_COMBINE_DT(MLA_DTYPE_BF16);
+  else
+    MLA_COMBINE_DT(MLA_DTYPE_F16);
+#undef MLA_COMBINE_DT
 #undef MLA_COMBINE
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MLA_ERR_HIP, std::string("combine launch failed: ") + hipGetErrorString(e));
