@@ -216,7 +216,12 @@ def quantize_kv_cache(kv_cache: torch.Tensor) -> Fp8KVCache:
     if kv_cache.dtype != torch.bfloat16 or kv_cache.shape[-1] != MLA_DIM_QK or kv_cache.shape[1] != _lib.MLA_PAGE_TOKENS:
         raise ValueError("kv_cache must be a bf16 [num_blocks, 64, 1, 576] tensor")
     nb = kv_cache.shape[0]
-    dst = fp8_kv_cache(nb, kv_cache.device)
+    # every code, scale and rope row is written below: no fill (three launches and a pass over the
+    # cache; 138496 tokens: 65.6 -> 50.7 us)
+    page, dev = _lib.MLA_PAGE_TOKENS, kv_cache.device
+    dst = Fp8KVCache(torch.empty(nb, page, MLA_DIM_V, dtype=torch.uint8, device=dev),
+                     torch.empty(nb, 4, page, dtype=torch.float32, device=dev),
+                     torch.empty(nb, page, MLA_DIM_QK - MLA_DIM_V, dtype=torch.bfloat16, device=dev))
     table = torch.arange(nb, dtype=torch.int32, device=kv_cache.device).reshape(nb, 1)
     lens = torch.zeros(nb, dtype=torch.int32, device=kv_cache.device)
     kv_append(kv_cache.reshape(nb, _lib.MLA_PAGE_TOKENS, MLA_DIM_QK), dst, table, lens)
