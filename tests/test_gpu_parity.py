@@ -387,6 +387,20 @@ def test_schedule_device_matches_host(gpu):
             assert torch.equal(s_d.cpu(), s_h) and torch.equal(n_d.cpu(), n_h)
 
 
+@pytest.mark.parametrize("lengths", [[64 * 17], [64 * 18], [64 * 256], [64 * 1024 + 1], [40000, 3, 40000], [5, 900000, 0, 64],
+                                     [64 * 40] * 3 + [100] * 70 + [300000], [9000] * 20])
+def test_schedule_long_sequences(gpu, lengths):
+    """Sequences that begin many parts, whose records the whole wave writes: one past the number that
+    a lane writes alone, one past a wave's width, several of them, and too many to be worth it."""
+    seq = torch.tensor(lengths, dtype=torch.int32, device=gpu)
+    for parts, fo in ((16, -1), (17, -1), (256, -1), (1024, -1), (1024, 0), (300, 5)):
+        say(f"schedule long B={len(lengths)} parts={parts} fo={fo}")
+        s_d, n_d = get_mla_metadata(seq, 16, 1, num_parts=parts, fixed_overhead=fo)
+        s_h, n_h = get_mla_metadata_host(lengths, parts, fo)
+        torch.cuda.synchronize()
+        assert torch.equal(s_d.cpu(), s_h) and torch.equal(n_d.cpu(), n_h)
+
+
 def test_flash_mla_call_shape(gpu):
     cfg = small_cfg("flash", 2, 1, 16, [100, 2000])
     inp = make_inputs(cfg, seed=11).to(gpu)
