@@ -1751,7 +1751,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
   constexpr bool kPtEarly = HT == 2;    // PV's first P^T fragments read at the end of QK
   constexpr bool kPrepEarly = HT == 2;  // stage k + 2's loads prepared at the end of iteration k - 1
   constexpr float kTau = ref_tau<DT>();
-  constexpr float kMinRef = -3.4028234664e38f;
+  constexpr float kMinRef = KV8 ? -3.4028234664e38f : -INFINITY;  // see m_ref
   constexpr int kPBytes = RT * 1024;
   __shared__ __attribute__((aligned(1024))) uint8_t lat_raw[kWideLat * kLatStageBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t rope_raw[kWideRope * kRopeStageBytes];
@@ -1995,8 +1995,10 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
     f32x4 o[WDT][RT];
     // row sums of this wave's QK rows: l_part over P as rounded for PV (normalises the
     // output), l_exact over the fp32 P (gives the lse)
-    // The reference max is kept finite (at least -FLT_MAX): a row without a key so far then needs no
-    // case of its own, since 2^(-inf - m) is 0 and any finite score lies more than tau above.
+    // KV8: the reference max is kept finite (at least -FLT_MAX): a row without a key so far then needs
+    // no case of its own, since 2^(-inf - m) is 0 and any finite score lies more than tau above, and
+    // no second copy of the reference is live in the stage loop.  The 16-bit forms have the
+    // registers for it, and are 0.2% faster with it.
     float m_ref[HT], l_part[HT], l_exact[HT];
     // The loads of one stage: wave w fetches row group w, 8 latent blocks and 1 rope block (one
     // global_load_lds_dwordx4 each, eight lanes per 128-byte line).  `prepare` does the scalar
@@ -2370,11 +2372,12 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         uint8_t LDS_AS* pw = ptb + (k & 1) * kPBytes + lane * 16;
 #pragma unroll
         for (int ht = 0; ht < HT; ++ht) {
+          const float mu = !KV8 && m_ref[ht] == -INFINITY ? 0.f : m_ref[ht];
           float pv[2][4];
 #pragma unroll
           for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pv[tt][r] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - m_ref[ht]);
+            for (int r = 0; r < 4; ++r) pv[tt][r] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - mu);
           const i32x4 pb = i32x4{(int)pack2<DT>(pv[0][0], pv[0][1]), (int)pack2<DT>(pv[0][2], pv[0][3]),
                                  (int)pack2<DT>(pv[1][0], pv[1][1]), (int)pack2<DT>(pv[1][2], pv[1][3])};
           l_part[ht] = packed_sum<DT>(pb, l_part[ht]);
@@ -2397,12 +2400,15 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
                             const StageIssue& si, const LaneOffsets& lo, uint32_t vm,
                             bool& over) __attribute__((always_inline)) {
         uint8_t LDS_AS* pw = ptb + ((kp + 1) & 1) * kPBytes + lo.pt;
+        float mu[HT];
+#pragma unroll
+        for (int ht = 0; ht < HT; ++ht) mu[ht] = !KV8 && m_ref[ht] == -INFINITY ? 0.f : m_ref[ht];
         float pvv[HT][8];
         // softmax element e of the 8 * HT this lane owns: row tile e / 8, token tile (e / 4) % 2,
         // token 4g + e % 4 of it
         auto p_elem = [&](int e) __attribute__((always_inline)) {
           const int ht = e >> 3, tt = (e >> 2) & 1, r = e & 3;
-          pvv[ht][e & 7] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - m_ref[ht]);
+          pvv[ht][e & 7] = fast_exp2(acc[ht][tt][r] * p.scale_log2 - mu[ht]);
         };
         auto p_finish = [&](int ht) __attribute__((always_inline)) {
           const float* v = pvv[ht];
