@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "mla_decode_amd.h"
+#include "mla_dispatch.h"
 #include "mla_sched.h"
 
 namespace mla {
@@ -3893,7 +3894,7 @@ hipError_t launch_main_dt(const Variant& v, const mla::KParams& kp, int head_blo
     }
     if (v.ws) return launch_main<DT, 4, 1, 1, true, false, true>(kp, head_blocks, st);
     if (v.nw == 1) return launch_main<DT, 1, 2, 1, false, false, true>(kp, head_blocks, st);
-    if (wide_enabled())
+    if (wide_enabled() && mla::wide_takes_sparse(kp.kv_sp, kp.kr_sp))
       return v.ht == 1 ? launch_wide<DT, 1, true>(kp, head_blocks, st) : launch_wide<DT, 2, true>(kp, head_blocks, st);
     if (v.ht == 1) return launch_main<DT, 4, 1, 4, false, false, true>(kp, head_blocks, st);
     return launch_main<DT, 4, 2, 3, false, false, true>(kp, head_blocks, st);

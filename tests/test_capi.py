@@ -466,3 +466,23 @@ def test_walk_schedule_equals_serial_packing(tmp_path):
                     "-I", os.path.join(repo, "mlc_decode_amd", "csrc"), "-o", str(exe), str(src)], check=True)
     bad, walked = map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
     assert walked > 30000 and bad == 0
+
+
+def _run_cpp(tmp_path, name, body):
+    """Compile and run a C++ program over the library's own headers; its standard output."""
+    repo = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src, exe = tmp_path / f"{name}.cpp", tmp_path / name
+    src.write_text(body)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(repo, "include"),
+                    "-I", os.path.join(repo, "mlc_decode_amd", "csrc"), "-o", str(exe), str(src)], check=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++ to build the dispatch header")
+def test_sparse_page_strides_the_wide_kernel_takes(tmp_path):
+    # a page stride of 2^32 elements or more does not fit the wide sparse form's 32-bit factor:
+    # such a cache goes to the one-ring kernel, whose row addresses are 64-bit
+    strides = [0, 64 * 576, (1 << 32) - 8, 1 << 32, (1 << 32) + 8, 3 << 32]
+    calls = "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_sparse({a}ll, {b}ll));\n' for a in strides for b in strides)
+    got = _run_cpp(tmp_path, "strides", '#include <cstdio>\n#include "mla_dispatch.h"\nint main() {\n' + calls + "}\n")
+    assert [int(v) for v in got.split()] == [int(a < 1 << 32 and b < 1 << 32) for a in strides for b in strides]

@@ -146,3 +146,18 @@ def test_sparse_wide_index_windows(gpu, H, dtype, views, topk, forced):
     torch.cuda.synchronize()
     assert torch.all(out[1] == 0) and torch.all(lse[1] == float("-inf"))
     assert_parity(out, lse, ref_o, ref_l, f"sparse wide H={H} topk={topk}")
+
+
+@pytest.mark.parametrize("H", [16, 64, 128])
+def test_sparse_page_stride_past_32_bits(gpu, H):
+    """Pages 2^32 elements (8 GiB) apart: every row address is formed in 64 bits."""
+    stride = 1 << 32
+    q, kv, idx = sparse_case(2, H, 100, nb=2, seed=H + 3)
+    pool = torch.empty(stride + 64 * 576, dtype=torch.bfloat16, device="cuda").as_strided((2, 64, 1, 576), (stride, 576, 576, 1))
+    pool.copy_(kv)
+    say(f"sparse page stride H={H}")
+    out, lse = run_sparse(q, pool, idx)
+    del pool
+    torch.cuda.empty_cache()
+    ref_o, ref_l = R.decode_sparse(q, kv, idx, 576 ** -0.5)
+    assert_parity(out, lse, ref_o, ref_l, f"sparse page stride H={H}")
