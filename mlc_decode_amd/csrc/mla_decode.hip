@@ -3067,14 +3067,17 @@ __device__ __forceinline__ float merge_row16(const uint16_t* __restrict__ ws_o, 
 // four CUs instead of one.  A wave keeps kQueue quarter rows in flight in a register queue: the
 // loop, unrolled by kQueue, consumes split k from queue slot k % kQueue and reloads that slot
 // with split k + kQueue (an index past the last split is clamped to it), so consuming a slot
-// waits only for that slot's load.  The loop is issue-bound (one wave per SIMD; the queue depth
-// does not matter between 16 and 32), so a block whose splits are all live runs without the
-// per-split zeroing of surplus rows that the last block needs.  The lse of all splits (lane l
+// waits only for that slot's load.  One wave's loop is issue-bound (one wave per SIMD; the queue
+// depth does not matter between 16 and 32), so a block whose splits are all live runs without the
+// per-split zeroing of surplus rows that the last block needs, and long merges in small grids are
+// shared by four waves.  The lse of all splits (lane l
 // holds splits l, l + 64, ..) and the quarter's chunk scale come first; the weight of split k
-// times that scale is formed once, into kw[k] (0 past the last split).  Arithmetic per output
-// element is merge_splits_wave's operation for operation (the same per-lane order of the max
-// and the sum, the same butterfly, the same product w * s and fma chain in split order): the
-// result is bit-identical.  (An LDS-DMA ring in place of the queue was no faster.)
+// times that scale is formed once, into kw[k] (0 past the last split).  The weights and the lse are
+// merge_splits_wave's operation for operation (the same per-lane order of the max and the sum, the
+// same butterfly, the same product w * s).  Over all splits so is the fma chain in split order, and
+// the row is bit-identical; a wave that takes a range of them (below) starts its chain there, and
+// the row differs from merge_splits_wave's by the order of four fp32 sums.  (An LDS-DMA ring in place
+// of the queue was no faster.)
 constexpr int kDeepSplits = 256;
 constexpr int kDeepMaxRows = 16384;  // kDeepSplits * kDeepMaxRows KiB = 2^32 bytes
 constexpr int kQueue = 32;
@@ -3200,7 +3203,10 @@ __global__ __launch_bounds__(DEEP ? 64 * DEEP : 256) void mla_combine_kernel(con
   const int b = blockIdx.x;
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.y * W + (DEEP ? 0 : wave);
+  // DEEP: a vector value, although one row serves the whole workgroup.  As a scalar (blockIdx.y) the
+  // compiler waits for the whole queue of merge_many_splits before each block of it: 160 rows x 256
+  // splits 10.1 -> 10.8 us, x 128 6.1 -> 6.4.
+  const int row = blockIdx.y * W + threadIdx.x / (DEEP ? 64 * DEEP : 64);
   if (row >= rows) return;
   const int base = splits[b];
   const int n = splits[b + 1] - base;
@@ -3214,12 +3220,13 @@ __global__ __launch_bounds__(DEEP ? 64 * DEEP : 256) void mla_combine_kernel(con
     if (n > kFewSplits && n <= kDeepSplits) {  // uniform
       float acc2[2];
       const bool share = DEEP > 1 && n > kShareSplits;  // uniform
-      if (!share && wave != 0) return;
+      const int wave_u = DEEP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave);
+      if (!share && wave_u != 0) return;
       const int per = share ? ((n + 4 * DEEP - 1) / (4 * DEEP)) * 4 : n;  // whole fours: the weights are read so
-      const int lo = wave * per;
+      const int lo = wave_u * per;
       const int hi = lo + per < n ? lo + per : n;
       const float lse2 = merge_many_splits<DT, SCALED>(ws_o, ws_scale, ws_lse, base, n, rows, row, q, lane,
-                                                       smem + wave * kDeepLds, lo, hi, acc2);
+                                                       smem + wave_u * kDeepLds, lo, hi, acc2);
       if (share) {
         sum_sh[wave][0][lane] = acc2[0];
         sum_sh[wave][1][lane] = acc2[1];
@@ -4049,11 +4056,13 @@ bool combine_is_deep(const mla::KParams& k) {
 
 template <typename PT, bool SCALED = false>
 int launch_combine(const mla::KParams& k, const PT* part_o, int dtype, int copy_single, hipStream_t st) {
-  // Four waves share a quarter row's splits where its merge is long (more than 64) and the rows are
-  // so few that one wave each leaves most of the chip idle.  Combine alone, one -> four waves: 16
-  // rows x 256 splits 7.1 -> 4.9 us, 128 x 256 10.1 -> 9.1, 32 x 128 5.3 -> 4.3; but 128 x 64 splits
-  // 4.3 -> 5.0, 128 x 32 3.9 -> 4.9, 256 rows x 128 7.0 -> 8.9.
-  const bool share = (int64_t)k.batch * k.rows <= 128 && k.num_parts > mla::kShareSplits * (int64_t)k.batch;
+  // Four waves share a quarter row's splits where its merge is long (more than 64) and every quarter
+  // row has a CU to itself.  Combine in the call's kernel trace, one -> four waves: 16 rows x 256
+  // splits 7.0 -> 4.9 us, x 128 4.8 -> 3.9; 32 x 128 4.9 -> 4.0; 64 x 256 7.4 -> 6.0, x 128 5.0 ->
+  // 4.5, x 65 4.6 -> 4.0.  At 128 rows a CU holds two of these workgroups and they lose: x 256 splits
+  // 8.8 -> 10.1, x 128 5.5 -> 6.1, x 96 4.7 -> 5.8.
+  const bool share = 4 * (int64_t)k.batch * k.rows <= cu_count_current() &&
+                     k.num_parts > mla::kShareSplits * (int64_t)k.batch;
   const int deep = !(std::is_same<PT, uint16_t>::value && combine_is_deep(k)) ? 0 : share ? 4 : 1;
   const int W = deep ? 1 : 4;
   const dim3 grid(k.batch, (k.rows + W - 1) / W, deep ? 4 : 1);
@@ -4259,7 +4268,8 @@ int mla_combine_absorb(const mla_decode_args* args, const void* w_uv_blk, void* 
   if (combine_is_deep(kp)) {
     // long merges: the combine kernel's DEEP form writes the merged rows (bf16/fp16, as the
     // fused merge rounds them into LDS) and their lse, and the projection reads every row from
-    // `out`; v is bit-identical to the fused merge's
+    // `out`; v is bit-identical to the fused merge's, except where the combine shares a long merge
+    // among four waves (launch_combine), whose fp32 sums have another order
     const int rc2 = launch_combine<uint16_t, true>(kp, kp.ws_o, args->dtype, 0, (hipStream_t)stream);
     if (rc2 != MLA_OK) return rc2;
     a.premerged = 1;

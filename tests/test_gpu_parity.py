@@ -613,11 +613,12 @@ def test_kv_append_skips_unassigned_pages(gpu):
     assert torch.equal(c.cpu(), want_cache) and torch.equal(ln.cpu(), want_lens)
 
 
-@pytest.mark.parametrize("B,H", [(1, 16), (2, 160)])
+@pytest.mark.parametrize("B,H", [(1, 16), (1, 64), (1, 65), (2, 160)])
 @pytest.mark.parametrize("n", [9, 16, 17, 63, 64, 65, 129, 255, 256, 257])
 def test_many_split_merge_edges(gpu, B, H, n):
-    """Merges of n splits in the dim-quarter combine, one wave per quarter row (320 rows) or four
-    that share its splits (16 rows), at the edges of the queue, the ranges and its 256 splits."""
+    """Merges of n splits in the dim-quarter combine, one wave per quarter row (65 and 320 rows) or four
+    that share its splits (up to a row for every fourth of the 256 CUs), at the edges of the queue,
+    the ranges and its 256 splits."""
     cfg = small_cfg(f"merge_{n}", B, 1, H, [64 * n, 64 * n - 63][:B])
     inp = make_inputs(cfg, seed=n)
     say(f"many-split merge B={B} H={H} n={n}")
