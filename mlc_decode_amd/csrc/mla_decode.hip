@@ -3594,13 +3594,10 @@ __global__ __launch_bounds__(kMetaThreads) void mla_metadata_kernel(
     block_exclusive_scan(cost, red_sh, &b64);
     total = b64;
   }
+  // (a 32-bit division on the walk path, in a branch of its own, made the kernel slower: 256 sequences
+  // of 2000 tokens 20.6 -> 21.8 us, 128 x 2048 12.4 -> 13.0, 64 x 4096 8.1 -> 8.3)
   int64_t lo, hi;
-  if (walk) {  // 32 bits: a 64-bit division is some hundred dependent instructions
-    lo = (int64_t)(((uint32_t)total32 + (uint32_t)num_parts - 1u) / (uint32_t)num_parts);
-    hi = lo + f;
-  } else {
-    payload_bounds(total, num_parts, f, &lo, &hi);
-  }
+  payload_bounds(total, num_parts, f, &lo, &hi);
   const int ncand = min_payload ? (int)(hi - lo) + 1 : 1;  // <= kMetaMaxCand (host-checked)
   int best = ncand - 1;  // the largest candidate (hi) always fits
   int64_t T;
@@ -3671,8 +3668,8 @@ __global__ __launch_bounds__(kMetaThreads) void mla_metadata_kernel(
       const int pinc = wave_inclusive_scan(inc);  // part increments of the resets up to this lane
       // pack_sequence_emit32, with the records of a sequence that begins many parts (a long one in
       // a small batch) written by the whole wave: one lane alone takes ~0.1 us a record.  One
-      // sequence of 32768 tokens in 256 parts 33.6 -> 4.8 us, 100000 in 1024 94 -> 5.9, four ragged
-      // ones 15.0 -> 6.7; 64 x 4096 tokens, where no sequence is long, 8.3 -> 8.5.
+      // sequence of 32768 tokens in 256 parts 32.2 -> 4.6 us, 100000 in 1024 90 -> 5.6, four of 20000
+      // 11.6 -> 5.4; 64 x 4096 tokens, where no sequence is long, 8.2 -> 8.1, 1024 x 500 33.3 -> 33.5.
       int first = 0, page0 = 0, split0 = 0, k = 0;  // the parts first .. first + k begin in the sequence
       if (in) {
         const int A = Sm - Sprev;
