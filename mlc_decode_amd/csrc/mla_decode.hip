@@ -3666,29 +3666,21 @@ __global__ __launch_bounds__(kMetaThreads) void mla_metadata_kernel(
       const int Sprev = below != 0 ? s_sh[win * kWalkWin + 63 - __builtin_clzll(below)] : e.rs;
       const int inc = ((mask >> lane) & 1) ? walk_parts(Sm - Sprev, Tb, f, c) + 1 : 0;
       const int pinc = wave_inclusive_scan(inc);  // part increments of the resets up to this lane
-      // pack_sequence_emit32, with the records of a sequence that begins many parts (a long one in
-      // a small batch) written by the whole wave: one lane alone takes ~0.1 us a record.  One
-      // sequence of 32768 tokens in 256 parts 32.2 -> 4.6 us, 100000 in 1024 90 -> 5.6, four of 20000
-      // 11.6 -> 5.4; 64 x 4096 tokens, where no sequence is long, 8.2 -> 8.1, 1024 x 500 33.3 -> 33.5.
-      int first = 0, page0 = 0, split0 = 0, k = 0;  // the parts first .. first + k begin in the sequence
+      // The records of a sequence that begins many parts (a long one in a small batch) are written by the
+      // whole wave: one lane alone takes ~0.1 us a record.  One sequence of 32768 tokens in 256 parts
+      // 32.2 -> 4.6 us, 100000 in 1024 90 -> 5.6, four of 20000 11.6 -> 5.4; 64 x 4096 tokens, where no
+      // sequence is long, 8.2 -> 8.1, 1024 x 500 33.3 -> 33.5.
+      SequenceCut q{false, 0, 0, 0, 1};
+      int first = 0;  // the parts first .. first + q.k begin in the sequence
       if (in) {
         const int A = Sm - Sprev;
         const int part = e.p + pinc - inc + walk_parts(A, Tb, f, c);
-        const int remain = walk_remain(A, Tb, f, c);
-        const int n = s_sh[m + 1] - Sm - f;
-        int slots = 1;
-        if (remain < n + f) {
-          const int take0 = remain - f;
-          page0 = take0 > 0 ? take0 : 0;
-          split0 = take0 > 0 ? 1 : 0;
-          first = part + 1;
-          const int left = n - page0;
-          if (Tb < left + f) k = (int)(((uint32_t)left + (uint32_t)c - 1u) / (uint32_t)c) - 1;
-          slots = split0 + k + 1;
-          emit(first, m, page0, split0);
-        }
-        splits[m + 1] = part + m - (e.w + __builtin_popcountll(below)) + slots;
+        q = cut_sequence32(s_sh[m + 1] - Sm - f, Tb, f, c, walk_remain(A, Tb, f, c));
+        first = part + 1;
+        if (q.cut) emit(first, m, q.page, q.split);
+        splits[m + 1] = part + m - (e.w + __builtin_popcountll(below)) + q.slots;
       }
+      const int k = q.k, page0 = q.page, split0 = q.split;
       // the lanes' own loops run side by side and the wave-wide ones in turn, so a sequence is taken
       // by the wave where it is long against their number
       const int n_long = __builtin_popcountll(__ballot(k > kEmitAlone));

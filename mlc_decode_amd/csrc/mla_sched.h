@@ -129,32 +129,27 @@ MLA_HD inline bool pack_sequence32(int n, int T, int f, int& remain, int& part, 
   return ok;
 }
 
-// pack_sequence with the part records, in 32-bit arithmetic, for payloads T >= f + 1 with
-// T + n + f < 2^31 (the device's parallel schedule): the same rule and the same records.
-template <class Emit>
-MLA_HD inline void pack_sequence_emit32(int b, int n, int T, int f, int& remain, int& part, int& cum,
-                                        const Emit& emit) {
-  if (remain >= n + f) {
-    remain -= n + f;
-    cum += 1;
-    return;
+// The records of one sequence of n pages that meets `remain` unused pages of payload, in 32-bit
+// arithmetic, for payloads T >= f + 1 (c = T - f) with T + n + f < 2^31: pack_sequence's rule, for the
+// device's parallel schedule and its host emulation alike.  cut: the sequence does not fit; then
+// a part begins inside it at page `page` (slot `split`), and k more after it, c pages and one slot
+// apart.  slots: workspace slots it takes.
+struct SequenceCut {
+  bool cut;
+  int32_t page, split, k, slots;
+};
+MLA_HD inline SequenceCut cut_sequence32(int n, int T, int f, int c, int remain) {
+  SequenceCut s{false, 0, 0, 0, 1};
+  if (remain < n + f) {
+    const int take0 = remain - f;
+    s.cut = true;
+    s.page = take0 > 0 ? take0 : 0;
+    s.split = take0 > 0 ? 1 : 0;
+    const int left = n - s.page;
+    if (T < left + f) s.k = (int)(((uint32_t)left + (uint32_t)c - 1u) / (uint32_t)c) - 1;
+    s.slots = s.split + s.k + 1;
   }
-  const int take0 = remain - f;
-  const int page = take0 > 0 ? take0 : 0;
-  const int split0 = take0 > 0 ? 1 : 0;
-  part += 1;
-  emit(part, b, page, split0);
-  int left = n - page;
-  int k = 0;
-  if (T < left + f) {
-    const uint32_t c = (uint32_t)(T - f);
-    k = (int)(((uint32_t)left + c - 1u) / c) - 1;
-    for (int j = 1; j <= k; ++j) emit(part + j, b, page + j * (int)c, split0 + j);
-    part += k;
-    left -= k * (int)c;
-  }
-  remain = T - left - f;
-  cum += split0 + k + 1;
+  return s;
 }
 
 // Sum over sequences of pages + f, and the payload bounds [lo, hi]: no packing fits num_parts
@@ -442,9 +437,10 @@ inline int schedule_walk_host(const int32_t* seqlens, int batch, int num_parts, 
     const int win = m / kWalkWin, lane = m % kWalkWin;
     const PackState st = walk_state(S, m, ent[best * nwin + win],
                                     msk[best * nwin + win] & ((1ull << lane) - 1), T, f, c);
-    int remain = (int)st.remain, part = st.part, cum = st.cum;
-    pack_sequence_emit32(m, S[m + 1] - S[m] - f, T, f, remain, part, cum, emit);
-    num_splits[m + 1] = cum;
+    const SequenceCut q = cut_sequence32(S[m + 1] - S[m] - f, T, f, c, (int)st.remain);
+    if (q.cut)
+      for (int j = 0; j <= q.k; ++j) emit(st.part + 1 + j, m, q.page + j * c, q.split + j);
+    num_splits[m + 1] = st.cum + q.slots;
   }
   for (int p = last + 1; p < num_parts; ++p) sched_write(sched + p * kSchedWords, batch, 0, batch, 0, 0);
   return num_splits[batch];
