@@ -117,7 +117,7 @@ def grown_workspace_size(current: Optional[int], need: int) -> int:
     return size
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)  # by type: 64.0 equals 64, but is refused
 def num_parts_for(batch: int, s_q: int, heads_q: int, heads_k: int = 1, cu_count: int = 0) -> int:
     """Schedule parts the decode kernel is laid out for (``mla_num_parts``)."""
     n = _lib.load().mla_num_parts(batch, s_q, heads_q, heads_k, cu_count)

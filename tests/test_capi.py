@@ -13,7 +13,7 @@ import torch
 
 from mlc_decode_amd import _lib
 from mlc_decode_amd._lib import MlaDecodeArgs, MlaKvAppendArgs
-from mlc_decode_amd.api import get_mla_metadata_host
+from mlc_decode_amd.api import get_mla_metadata_host, num_parts_for
 from oracle import mla_ref as R
 
 HEADER = os.path.join(os.path.dirname(os.path.dirname(__file__)), "include", "mla_decode_amd.h")
@@ -466,6 +466,14 @@ def test_walk_schedule_equals_serial_packing(tmp_path):
                     "-I", os.path.join(repo, "mlc_decode_amd", "csrc"), "-o", str(exe), str(src)], check=True)
     bad, walked = map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
     assert walked > 30000 and bad == 0
+
+
+def test_num_parts_refuses_non_integers_whatever_came_before():
+    # 64 and 64.0 compare equal: a remembered answer for one must not serve the other
+    assert num_parts_for(64, 1, 128, 1, 256) == num_parts_for(64, 1, 128, 1, 256)
+    for args in ((64.0, 1, 128, 1, 256), (64, 1.0, 128, 1, 256), (64, 1, 128, 1, 256.0)):
+        with pytest.raises(ctypes.ArgumentError):
+            num_parts_for(*args)
 
 
 def _run_cpp(tmp_path, name, body):
