@@ -2731,8 +2731,12 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
 #pragma unroll 4
         for (int j = 0; j < R / 4; ++j) *(i32x4*)(dst + j * stride) = staged(j);
       } else {
+        // sparse, and fp8 above 64 rows: whole groups of padding rows are left out (132 sequences x 72
+        // heads, top 128: 27.9 -> 26.0 us, one-ring 26.7).  The dense forms and the 64-row fp8 form
+        // store them: those without padding lost more than the others gained, or nothing was gained.
+        const int nj = (SPARSE || (KV8 && HT == 2)) && p.rows - rowb < R ? (p.rows - rowb + 3) / 4 : R / 4;
 #pragma unroll 2
-        for (int j = 0; j < R / 4; ++j) {
+        for (int j = 0; j < nj; ++j) {
           int row = rowb + 4 * j + r0;
           row = row < p.rows ? row : p.rows - 1;  // padding rows repeat the last row's values
           uint16_t* dst;
@@ -3839,9 +3843,10 @@ hipError_t launch_main(const mla::KParams& kp, int head_blocks, hipStream_t st) 
 }
 
 // The 64- and 128-row decodes over a 16-bit cache run the wide kernel (PV split by dims across the
-// waves) unless MLA_WIDE=0 selects the one-ring four-wave kernel, and so do those over the paged fp8
-// cache; the sparse decode over it keeps the one-ring kernel (its three row addresses per lane do
-// not fit the 128-row form).
+// waves) unless MLA_WIDE=0 selects the one-ring four-wave kernel, and so do the sparse decode and that
+// over the paged fp8 cache where their segments are long enough (mla_dispatch.h); the sparse decode
+// over the fp8 cache keeps the one-ring kernel (its three row addresses per lane do not fit the
+// 128-row form).
 bool wide_enabled() {
   static std::once_flag once;
   static bool on = true;
@@ -3890,7 +3895,8 @@ hipError_t launch_main_dt(const Variant& v, const mla::KParams& kp, int head_blo
     }
     if (v.ws) return launch_main<DT, 4, 1, 1, true, false, true>(kp, head_blocks, st);
     if (v.nw == 1) return launch_main<DT, 1, 2, 1, false, false, true>(kp, head_blocks, st);
-    if (wide_enabled() && mla::wide_takes_sparse(kp.kv_sp, kp.kr_sp))
+    if (wide_enabled() &&
+        mla::wide_takes_sparse(kp.rows, kp.batch, kp.topk, kp.num_parts, cu_count_current(), kp.kv_sp, kp.kr_sp))
       return v.ht == 1 ? launch_wide<DT, 1, true>(kp, head_blocks, st) : launch_wide<DT, 2, true>(kp, head_blocks, st);
     if (v.ht == 1) return launch_main<DT, 4, 1, 4, false, false, true>(kp, head_blocks, st);
     return launch_main<DT, 4, 2, 3, false, false, true>(kp, head_blocks, st);
@@ -3899,7 +3905,8 @@ hipError_t launch_main_dt(const Variant& v, const mla::KParams& kp, int head_blo
     if (kp.kv_scale != nullptr) {  // fp8 latent cache
       if (v.ws) return launch_main<DT, 4, 1, 1, true, true>(kp, head_blocks, st);
       if (v.nw == 1) return launch_main<DT, 1, 2, 1, false, true>(kp, head_blocks, st);
-      if (wide_enabled() && kp.ks_sb < (1 << 28)) {  // a lane's scale offset is formed in 32 bits
+      if (wide_enabled() &&
+          mla::wide_takes_fp8(kp.rows, kp.batch, kp.bt_width, kp.num_parts, cu_count_current(), kp.ks_sb)) {
         if (v.ht == 1) launch_wide_form<DT, 1, false, false, true>(kp, head_blocks, st);
         else launch_wide_form<DT, 2, false, false, true>(kp, head_blocks, st);
         return hipGetLastError();

@@ -486,11 +486,34 @@ def _run_cpp(tmp_path, name, body):
     return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
 
 
+_DISPATCH_PROG = '#include <cstdio>\n#include "mla_dispatch.h"\nint main() {\n%s}\n'
+
+
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++ to build the dispatch header")
 def test_sparse_page_strides_the_wide_kernel_takes(tmp_path):
     # a page stride of 2^32 elements or more does not fit the wide sparse form's 32-bit factor:
     # such a cache goes to the one-ring kernel, whose row addresses are 64-bit
     strides = [0, 64 * 576, (1 << 32) - 8, 1 << 32, (1 << 32) + 8, 3 << 32]
-    calls = "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_sparse({a}ll, {b}ll));\n' for a in strides for b in strides)
-    got = _run_cpp(tmp_path, "strides", '#include <cstdio>\n#include "mla_dispatch.h"\nint main() {\n' + calls + "}\n")
+    calls = "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_sparse(128, 64, 2048, 256, 256, {a}ll, {b}ll));\n'
+                    for a in strides for b in strides)
+    got = _run_cpp(tmp_path, "strides", _DISPATCH_PROG % calls)
     assert [int(v) for v in got.split()] == [int(a < 1 << 32 and b < 1 << 32) for a in strides for b in strides]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++ to build the dispatch header")
+def test_short_segments_stay_off_the_wide_kernel(tmp_path):
+    # both sides of each line of the sparse and fp8 rules, 256 CUs: (rows, batch, top-k or table
+    # width, parts, wide?)
+    sparse = [(64, 1, 512, 256, 1), (40, 16, 64, 256, 1), (40, 17, 64, 256, 0), (64, 64, 64, 256, 0), (64, 64, 256, 256, 0),
+              (64, 64, 512, 256, 1), (40, 132, 128, 256, 0), (40, 132, 256, 256, 1), (64, 8, 1536, 256, 0), (64, 8, 2048, 256, 1),
+              (64, 100, 192, 100, 0), (64, 100, 193, 100, 1), (72, 15, 64, 256, 1), (72, 16, 64, 256, 0), (100, 128, 64, 256, 0),
+              (100, 129, 64, 256, 1), (72, 64, 65, 256, 1), (128, 64, 64, 256, 1), (150, 64, 64, 256, 1)]
+    fp8 = [(64, 64, 8, 256, 0), (64, 64, 16, 256, 1), (40, 132, 4, 256, 0), (40, 132, 8, 256, 1), (64, 256, 6, 256, 1),
+           (64, 256, 5, 256, 0), (40, 1, 8, 2, 1), (40, 1, 8, 4, 0), (64, 1, 8, 4, 1), (64, 1, 8, 8, 0), (64, 1, 256, 256, 0),
+           (72, 64, 1, 256, 0), (72, 64, 2, 256, 1), (128, 1, 1, 256, 1), (200, 32, 1, 128, 1)]
+    calls = "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_sparse({r}, {b}, {k}, {n}, 256, 36864, 36864));\n'
+                    for r, b, k, n, _ in sparse)
+    calls += "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_fp8({r}, {b}, {w}, {n}, 256, {sb}ll));\n'
+                     for sb in (64, 1 << 28) for r, b, w, n, _ in fp8)
+    got = [int(v) for v in _run_cpp(tmp_path, "segments", _DISPATCH_PROG % calls).split()]
+    assert got == [c[-1] for c in sparse] + [c[-1] for c in fp8] + [0] * len(fp8)
