@@ -237,17 +237,12 @@ def _check_native_cache(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
         raise ValueError("kv cache must be [num_blocks, 64, 1, D] with unit stride in D")
 
 
-def _split_kv(kv_cache) -> Tuple[torch.Tensor, torch.Tensor]:
-    if isinstance(kv_cache, Fp8KVCache):
-        raise ValueError("an fp8 cache has no bf16 latent half")
-    if isinstance(kv_cache, (tuple, list)):
-        latent, rope = kv_cache
-        if latent.shape[-1] != MLA_DIM_V or rope.shape[-1] != MLA_DIM_QK - MLA_DIM_V:
-            raise ValueError("kv pair must be (latent [..., 512], rope [..., 64])")
-        return latent, rope
-    if kv_cache.shape[-1] != MLA_DIM_QK:
-        raise ValueError(f"kv_cache last dim must be {MLA_DIM_QK}")
-    return kv_cache[..., :MLA_DIM_V], kv_cache[..., MLA_DIM_V:]
+def _split_kv(kv_pair) -> Tuple[torch.Tensor, torch.Tensor]:
+    """A cache given as two tensors: ``(latent [..., 512], rope [..., 64])``."""
+    latent, rope = kv_pair
+    if latent.shape[-1] != MLA_DIM_V or rope.shape[-1] != MLA_DIM_QK - MLA_DIM_V:
+        raise ValueError("kv pair must be (latent [..., 512], rope [..., 64])")
+    return latent, rope
 
 
 def make_decode_args(q: torch.Tensor, kv_cache, block_table: Optional[torch.Tensor],
@@ -555,7 +550,8 @@ def kv_append(kv_new: torch.Tensor, kv_cache, block_table: torch.Tensor,
     a = MlaKvAppendArgs.from_buffer_copy(_APPEND_ARGS.pack(
         B, n_new, _DTYPES[kv_new.dtype], latent.shape[0], kv_new.data_ptr(), new_b, new_t,
         latent.data_ptr(), rope.data_ptr() + rope_offset, kv_page, kv_tok, kr_page, kr_tok,
-        block_table.data_ptr(), block_table.stride(0) if B > 1 else min(block_table.stride(0), 2 ** 31 - 1), block_table.shape[1], cache_seqlens.data_ptr(),
+        block_table.data_ptr(), block_table.stride(0) if B > 1 else min(block_table.stride(0), 2 ** 31 - 1),
+        block_table.shape[1], cache_seqlens.data_ptr(),
         status.data_ptr() if status is not None else 0, *scale_args))
     check("mla_kv_append", _lib.load().mla_kv_append(ctypes.byref(a), _stream_ptr(kv_new.device)))
     return a
