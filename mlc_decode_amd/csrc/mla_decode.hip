@@ -4050,6 +4050,14 @@ bool combine_is_deep(const mla::KParams& k) {
   return k.num_parts >= 16 * k.batch && k.rows <= mla::kDeepMaxRows;
 }
 
+// The most pages a sequence can have, as far as the host knows: an index list's length, the table's
+// width, or a batch stride's worth of tokens of a contiguous cache.
+int64_t pages_bound(const mla::KParams& k) {
+  if (k.indices != nullptr) return (k.topk + mla::kPageTokens - 1) / mla::kPageTokens;
+  if (k.block_table != nullptr) return k.bt_width;
+  return k.kv_st > 0 ? k.kv_sb / (k.kv_st * mla::kPageTokens) : 0;
+}
+
 template <typename PT, bool SCALED = false>
 int launch_combine(const mla::KParams& k, const PT* part_o, int dtype, int copy_single, hipStream_t st) {
   // Four waves share a quarter row's splits where its merge is long (more than 64) and every quarter
@@ -4057,8 +4065,10 @@ int launch_combine(const mla::KParams& k, const PT* part_o, int dtype, int copy_
   // splits 7.0 -> 4.9 us, x 128 4.8 -> 3.9; 32 x 128 4.9 -> 4.0; 64 x 256 7.4 -> 6.0, x 128 5.0 ->
   // 4.5, x 65 4.6 -> 4.0.  At 128 rows a CU holds two of these workgroups and they lose: x 256 splits
   // 8.8 -> 10.1, x 128 5.5 -> 6.1, x 96 4.7 -> 5.8.
+  // Where no sequence can have so many pages the extra waves only start and end (one sequence x 64
+  // heads x 165 tokens, the whole call: 13.76 -> 13.89).
   const bool share = 4 * (int64_t)k.batch * k.rows <= cu_count_current() &&
-                     k.num_parts > mla::kShareSplits * (int64_t)k.batch;
+                     k.num_parts > mla::kShareSplits * (int64_t)k.batch && pages_bound(k) > mla::kShareSplits;
   const int deep = !(std::is_same<PT, uint16_t>::value && combine_is_deep(k)) ? 0 : share ? 4 : 1;
   const int W = deep ? 1 : 4;
   const dim3 grid(k.batch, (k.rows + W - 1) / W, deep ? 4 : 1);
