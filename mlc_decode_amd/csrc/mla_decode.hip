@@ -4051,11 +4051,11 @@ bool combine_is_deep(const mla::KParams& k) {
 }
 
 // The most pages a sequence can have, as far as the host knows: an index list's length, the table's
-// width, or a batch stride's worth of tokens of a contiguous cache.
+// width, or what the strides of a contiguous cache tell.
 int64_t pages_bound(const mla::KParams& k) {
   if (k.indices != nullptr) return (k.topk + mla::kPageTokens - 1) / mla::kPageTokens;
   if (k.block_table != nullptr) return k.bt_width;
-  return k.kv_st > 0 ? k.kv_sb / (k.kv_st * mla::kPageTokens) : 0;
+  return mla::contiguous_pages_bound(k.kv_sb, k.kv_st);
 }
 
 template <typename PT, bool SCALED = false>

@@ -1,5 +1,5 @@
-// mla_dispatch.h -- which decodes the wide kernel takes (host code, no HIP: the CPU tests compile
-// these rules by themselves).
+// mla_dispatch.h -- which decodes the wide kernel takes, and what bounds a sequence's pages (host code,
+// no HIP: the CPU tests compile these rules by themselves).
 //
 // The wide kernel (PV split by output dims) beats the one-ring kernel where a segment is long enough
 // to repay its start and end: a second ring to fill, P^T through LDS, rows staged through LDS on the
@@ -8,6 +8,14 @@
 #include <stdint.h>
 
 namespace mla {
+
+// The most pages a sequence of a contiguous cache can have: a batch stride's worth of tokens where the
+// sequences lie one after another.  A batch stride of less than a page of tokens belongs to another
+// order (token-major, or one sequence, whose batch stride is never used) and bounds nothing.
+inline int64_t contiguous_pages_bound(int64_t stride_batch, int64_t stride_tok) {
+  const int64_t page = 64 * stride_tok;
+  return page > 0 && stride_batch >= page ? (stride_batch + page - 1) / page : INT64_MAX;
+}
 
 // 65 .. 127 rows leave row tiles of a workgroup empty; with one-page sequences on up to half of the
 // CUs nothing makes up for it (top 64: 32 sequences x 72 heads 23.2 -> 24.3, 64 x 100 heads 25.4 ->

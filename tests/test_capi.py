@@ -517,3 +517,15 @@ def test_short_segments_stay_off_the_wide_kernel(tmp_path):
                      for sb in (64, 1 << 28) for r, b, w, n, _ in fp8)
     got = [int(v) for v in _run_cpp(tmp_path, "segments", _DISPATCH_PROG % calls).split()]
     assert got == [c[-1] for c in sparse] + [c[-1] for c in fp8] + [0] * len(fp8)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++ to build the dispatch header")
+def test_contiguous_pages_bound(tmp_path):
+    # (batch stride, token stride, pages): sequence-major caches give their length; token-major ones, a
+    # broadcast cache and one sequence of any batch stride give no bound
+    big = 2 ** 63 - 1
+    cases = [(64 * 65 * 512, 512, 65), (64 * 64 * 512 + 512, 512, 65), (64 * 64 * 512, 512, 64), (64 * 512, 512, 1),
+             (512, 4 * 512, big), (0, 512, big), (63 * 512, 512, big), (0, 0, big), (8, 0, big)]
+    calls = "".join(f'  std::printf("%lld\\n", (long long)mla::contiguous_pages_bound({b}ll, {t}ll));\n' for b, t, _ in cases)
+    got = _run_cpp(tmp_path, "contiguous", _DISPATCH_PROG % calls)
+    assert [int(v) for v in got.split()] == [c[2] for c in cases]
