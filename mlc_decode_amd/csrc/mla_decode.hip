@@ -2034,10 +2034,14 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       const bool real = k < nst;
       const int st = st_begin + (real ? k : nst - 1);
       StageIssue si;
-      si.lat_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
-          (int)(uint32_t)(uintptr_t)(lat + (k % kWideLat) * kLatStageBytes + wave * 8 * 1024));
-      si.rope_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
-          (int)(uint32_t)(uintptr_t)(rope + (k % kWideRope) * kRopeStageBytes + wave * 1024));
+      // Dense 16-bit forms: after the addresses.  (Before them the compiler keeps more scalars live: 132
+      // ragged sequences x 64 heads 69.0 -> 69.4 us, 8 x 300 tokens x 64 heads 16.28 -> 16.40.)
+      const auto set_dst = [&]() __attribute__((always_inline)) {
+        si.lat_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(lat + (k % kWideLat) * kLatStageBytes + wave * 8 * 1024));
+        si.rope_dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(rope + (k % kWideRope) * kRopeStageBytes + wave * 1024));
+      };
       const auto uni64 = [](const char* q) {
         const uint64_t v = (uint64_t)(uintptr_t)q;
         return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32) |
@@ -2071,6 +2075,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         return si;
       }
       if constexpr (SPARSE) {
+        set_dst();
         const int ks = real ? k : (nst > 0 ? nst - 1 : 0);
         if (ks - win0 >= kSparseWin) load_window(ks);  // uniform
         const int ln = fresh_lane();
@@ -2117,6 +2122,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
       const uint32_t cl = real ? (uint32_t)(((lane & 7) ^ stage_swz(((wave & 1) << 3) | (lane >> 3))) << 4) : 0u;
       si.on = (uint32_t)(row * kv_st) * 2 + cl;
       si.orp = FUSED ? si.on : (uint32_t)(row * kr_st) * 2 + cl;
+      set_dst();
       return si;
     };
     auto issue_one = [&](const StageIssue& si, auto jtag) __attribute__((always_inline)) {
@@ -2514,7 +2520,7 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         } else {
           if constexpr (MODE == kPassFirstStageRef) {
 #pragma unroll
-            for (int ht = 0; ht < HT; ++ht) m_ref[ht] = fmaxf(wave_max_g(lmx[ht]), kMinRef);
+            for (int ht = 0; ht < HT; ++ht) m_ref[ht] = KV8 ? fmaxf(wave_max_g(lmx[ht]), kMinRef) : wave_max_g(lmx[ht]);
           }
           softmax_publish(0, acc);
         }
