@@ -3231,7 +3231,7 @@ __global__ __launch_bounds__(DEEP ? 64 * DEEP : 256) void mla_combine_kernel(con
       float acc2[2];
       const bool share = DEEP > 1 && n > kShareSplits;  // uniform
       const int wave_u = DEEP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave);
-      if (!share && wave_u != 0) return;
+      if (DEEP > 1 && !share && wave_u != 0) return;
       const int per = share ? ((n + 4 * DEEP - 1) / (4 * DEEP)) * 4 : n;  // whole fours: the weights are read so
       const int lo = wave_u * per;
       const int hi = lo + per < n ? lo + per : n;
@@ -3252,7 +3252,7 @@ __global__ __launch_bounds__(DEEP ? 64 * DEEP : 256) void mla_combine_kernel(con
       if (q == 0 && lane == 0 && lse_dst != nullptr) *lse_dst = lse2 * kLn2;
       return;
     }
-    if (q != 0 || wave != 0) return;
+    if (q != 0 || (DEEP > 1 && wave != 0)) return;
   }
   float acc[8];
   float lse2;
