@@ -2738,11 +2738,13 @@ __global__ __launch_bounds__(256, 1) void mla_wide_kernel(const int32_t* __restr
         for (int j = 0; j < R / 4; ++j) *(i32x4*)(dst + j * stride) = staged(j);
       } else {
         // sparse, and fp8 above 64 rows: whole groups of padding rows are left out (132 sequences x 72
-        // heads, top 128: 27.9 -> 26.0 us, one-ring 26.7).  The dense forms and the 64-row fp8 form
-        // store them: those without padding lost more than the others gained, or nothing was gained.
-        const int nj = (SPARSE || (KV8 && HT == 2)) && p.rows - rowb < R ? (p.rows - rowb + 3) / 4 : R / 4;
+        // heads, top 128: 28.9 -> 27.3 us, 132 x 40, top 1000: 45.4 -> 44.6).  The dense forms and the
+        // 64-row fp8 form store them: those without padding lost more than the others gained, or nothing
+        // was gained.  (As a loop of a run-time count the sparse forms without padding lost 0.2 to 0.4
+        // us; with each padding row left out by its lane nothing was gained.)
 #pragma unroll 2
-        for (int j = 0; j < nj; ++j) {
+        for (int j = 0; j < R / 4; ++j) {
+          if ((SPARSE || (KV8 && HT == 2)) && rowb + 4 * j >= p.rows) break;  // uniform
           int row = rowb + 4 * j + r0;
           row = row < p.rows ? row : p.rows - 1;  // padding rows repeat the last row's values
           uint16_t* dst;
