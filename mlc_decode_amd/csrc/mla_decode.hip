@@ -3680,8 +3680,8 @@ __global__ __launch_bounds__(kMetaThreads) void mla_metadata_kernel(
       const int pinc = wave_inclusive_scan(inc);  // part increments of the resets up to this lane
       // The records of a sequence that begins many parts (a long one in a small batch) are written by the
       // whole wave: one lane alone takes ~0.1 us a record.  One sequence of 32768 tokens in 256 parts
-      // 32.2 -> 4.6 us, 100000 in 1024 90 -> 5.6, four of 20000 11.6 -> 5.4; 64 x 4096 tokens, where no
-      // sequence is long, 8.2 -> 8.1, 1024 x 500 33.3 -> 33.5.
+      // 32.2 -> 4.6 us, 100000 in 1024 90 -> 5.6, four of 20000 11.6 -> 5.4; where no sequence is long, 64 x
+      // 4096 tokens 8.4 -> 8.3, 256 x 2000 20.7 -> 20.75, 1024 x 500 33.5 -> 33.8 (the test in each window).
       SequenceCut q{false, 0, 0, 0, 1};
       int first = 0;  // the parts first .. first + q.k begin in the sequence
       if (in) {
