@@ -3914,7 +3914,8 @@ hipError_t launch_main_dt(const Variant& v, const mla::KParams& kp, int head_blo
       if (v.ws) return launch_main<DT, 4, 1, 1, true, true>(kp, head_blocks, st);
       if (v.nw == 1) return launch_main<DT, 1, 2, 1, false, true>(kp, head_blocks, st);
       if (wide_enabled() &&
-          mla::wide_takes_fp8(kp.rows, kp.batch, kp.bt_width, kp.num_parts, cu_count_current(), kp.ks_sb)) {
+          mla::wide_takes_fp8(kp.rows, kp.heads, kp.batch, kp.bt_width, kp.num_parts, cu_count_current(),
+                              kp.ks_sb)) {
         if (v.ht == 1) launch_wide_form<DT, 1, false, false, true>(kp, head_blocks, st);
         else launch_wide_form<DT, 2, false, false, true>(kp, head_blocks, st);
         return hipGetLastError();

@@ -502,19 +502,23 @@ def test_sparse_page_strides_the_wide_kernel_takes(tmp_path):
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++ to build the dispatch header")
 def test_short_segments_stay_off_the_wide_kernel(tmp_path):
-    # both sides of each line of the sparse and fp8 rules, 256 CUs: (rows, batch, top-k or table
-    # width, parts, wide?)
-    sparse = [(64, 1, 512, 256, 1), (40, 16, 64, 256, 1), (40, 17, 64, 256, 0), (64, 64, 64, 256, 0), (64, 64, 256, 256, 0),
+    # both sides of each line of the sparse and fp8 rules, 256 CUs: (rows, batch, top-k, parts, wide?) and
+    # (rows, heads, batch, table width, parts, wide?)
+    sparse = [(64, 1, 512, 256, 1), (64, 16, 64, 256, 1), (64, 17, 64, 256, 0), (40, 1, 193, 256, 1), (40, 1, 192, 256, 0),
+              (39, 1, 512, 256, 0), (48, 2, 512, 256, 0), (64, 64, 64, 256, 0), (64, 64, 256, 256, 0),
               (64, 64, 512, 256, 1), (40, 132, 128, 256, 0), (40, 132, 256, 256, 1), (64, 8, 1536, 256, 0), (64, 8, 2048, 256, 1),
               (64, 100, 192, 100, 0), (64, 100, 193, 100, 1), (72, 15, 64, 256, 1), (72, 16, 64, 256, 0), (100, 128, 64, 256, 0),
               (100, 129, 64, 256, 1), (72, 64, 65, 256, 1), (128, 64, 64, 256, 1), (150, 64, 64, 256, 1)]
     fp8 = [(64, 64, 8, 256, 0), (64, 64, 16, 256, 1), (40, 132, 4, 256, 0), (40, 132, 8, 256, 1), (64, 256, 6, 256, 1),
            (64, 256, 5, 256, 0), (40, 1, 8, 2, 1), (40, 1, 8, 4, 0), (64, 1, 8, 4, 1), (64, 1, 8, 8, 0), (64, 1, 256, 256, 0),
            (72, 64, 1, 256, 0), (72, 64, 2, 256, 1), (128, 1, 1, 256, 1), (200, 32, 1, 128, 1)]
+    fp8 = [(c[0], *c) for c in fp8]  # one query token
+    fp8 += [(128, 64, 16, 1, 256, 0), (128, 64, 15, 1, 256, 1), (160, 40, 51, 1, 256, 0), (160, 40, 52, 1, 256, 1),
+            (144, 72, 38, 2, 256, 1), (256, 128, 38, 1, 256, 1), (160, 160, 38, 1, 256, 1)]
     calls = "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_sparse({r}, {b}, {k}, {n}, 256, 36864, 36864));\n'
                     for r, b, k, n, _ in sparse)
-    calls += "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_fp8({r}, {b}, {w}, {n}, 256, {sb}ll));\n'
-                     for sb in (64, 1 << 28) for r, b, w, n, _ in fp8)
+    calls += "".join(f'  std::printf("%d\\n", (int)mla::wide_takes_fp8({r}, {h}, {b}, {w}, {n}, 256, {sb}ll));\n'
+                     for sb in (64, 1 << 28) for r, h, b, w, n, _ in fp8)
     got = [int(v) for v in _run_cpp(tmp_path, "segments", _DISPATCH_PROG % calls).split()]
     assert got == [c[-1] for c in sparse] + [c[-1] for c in fp8] + [0] * len(fp8)
 
